@@ -12,15 +12,12 @@
 // Mapping: one lane per stream (DM row, multiplet m); a block holds 256/M DM rows. Each lane
 // walks its stream through time once. Every boxcar level keeps its last values in a register
 // window (Wmax and Dout are template parameters, so every shift, sum and candidate of one
-// output bin is unrolled at compile time). Each candidate is weighted as it is formed and
-// compared with the level's running best (strict '>', candidates visited in (isamp, p)
-// order), so the lane ends each bin with the exact first maximum per level. Levels are then
-// combined in order (strict '>'), and the multiplets of a DM row are reduced through LDS in
-// (level, m) order: the result is the reference's maximum and argmax token, bit for bit.
-//
-// Samples are staged through LDS in tiles of TL positions (coalesced 4-element loads);
-// tiles are aligned to output bins. Positions before the row start are read as zeros,
-// which equals the zero initial state of the windows.
+// output bin is unrolled at compile time). k_pf keeps the largest value of each profile and
+// finds the token of the winning stream in a second step (below); k_pf_var, which also forms
+// the optional float64 variances, weights and compares each candidate as it is formed (strict
+// '>', candidates visited in (isamp, p) order). Either way the multiplets of a DM row are
+// reduced in (level, m) order, and the result is the reference's maximum and argmax token, bit
+// for bit. Positions before the row start count as zeros, the initial state of the windows.
 //
 // The chunk's time axis is split into nseg segments (blockIdx.z), one workgroup each, so
 // that short chunks still fill the chip. A segment's lanes start from zero windows and run
@@ -40,9 +37,10 @@ namespace pirate_amd {
 
 static constexpr int kPfThreads = 256;
 static constexpr int kPfMaxDout = 32;
+static constexpr int kPfLine = 128;      // bytes of a row that one staging tile covers
 
-// Staging tile length (positions) for output time downsampling Dout: whole output bins, at
-// least kPfTileMin positions when Dout >= 4, 8 bins below.
+// k_pf_var's staging tile length (positions) for output time downsampling Dout: whole output
+// bins, at least kPfTileMin positions when Dout >= 4, 8 bins below.
 static constexpr int kPfTileMin = 16;
 __host__ __device__ constexpr int pf_tile_len(int dout)
 {
@@ -74,9 +72,9 @@ struct PfShape {
     static constexpr int win(int l) { return 3 * sgrid(l) + 1; }
     static constexpr int woff(int l) { return (l == 0) ? 0 : woff(l - 1) + win(l - 1); }
     static constexpr int WTOT = woff(NLEV);
-    // Occupancy target: 4 waves/SIMD (128 VGPRs) when the register windows are small,
-    // else 2 (the compiler's unrolled schedule would otherwise spill).
-    static constexpr int WAVES = (WTOT + P <= 32 && LD >= 2) ? 4 : 2;
+    // Waves per SIMD: 3 (168 VGPRs, as many as the LDS allows) where step 2's unrolled walk
+    // fits, else 2.
+    static constexpr int WAVES = (LD == 5 || (LD == 0 && LW >= 4) || (LD == 1 && LW == 5)) ? 2 : 3;
 };
 
 template<typename S, bool VAR>
@@ -231,15 +229,151 @@ struct PfLane {
     }
 };
 
+// The same walk without weights or codes: the largest value of every profile in a bin (the
+// weight of a profile is constant over a bin, and rounding is monotonic, so the largest
+// weighted candidate of a profile is its weight times this value, bit for bit).
+template<typename S>
+struct PfMax {
+    float w[S::WTOT];          // boxcar windows, as in PfLane
+    float mx[S::P];            // per profile: largest value in the current bin
+    bool nonfinite;            // an infinity or NaN entered the windows in the current bin
+
+    template<int L, int POS, bool EVAL>
+    __device__ __forceinline__ void levels()
+    {
+        if constexpr (L < S::NLEV) {
+            if constexpr ((POS + 1) % S::dt(L) == 0) {
+                constexpr int o = S::woff(L), s = S::sgrid(L), n = S::win(L);
+                if constexpr (L > 0) {
+                    constexpr int op = S::woff(L - 1), back = S::sgrid(L - 1);
+#pragma unroll
+                    for (int i = n - 1; i > 0; i--)
+                        w[o + i] = w[o + i - 1];
+                    w[o] = w[op + back] + w[op];
+                }
+                if constexpr (L == S::NLEV - 1)        // every sample enters one of these sums
+                    nonfinite |= !(fabsf(w[o]) < __builtin_inff());
+                if constexpr (EVAL) {
+                    constexpr bool first = (POS + 1) / S::dt(L) == 1;
+                    const float x3 = w[o], x2 = w[o + s], x1 = w[o + 2 * s], x0 = w[o + 3 * s];
+                    if constexpr (L == 0)
+                        mx[0] = first ? x3 : fmaxf(mx[0], x3);
+                    if constexpr (S::P > 1) {
+                        constexpr int p = 3 * L + 1;
+                        const float h3 = 0.5f * x3;
+                        const float y1 = x2 + x3;
+                        const float y2 = (0.5f * x1 + x2) + h3;
+                        const float y3 = ((0.5f * x0 + x1) + x2) + h3;
+                        mx[p] = first ? y1 : fmaxf(mx[p], y1);
+                        mx[p + 1] = first ? y2 : fmaxf(mx[p + 1], y2);
+                        mx[p + 2] = first ? y3 : fmaxf(mx[p + 2], y3);
+                    }
+                }
+                levels<L + 1, POS, EVAL>();
+            }
+        }
+    }
+
+    template<bool EVAL, int POS = 0>
+    __device__ __forceinline__ void bin(const float *xs)
+    {
+        if constexpr (POS < S::DOUT) {
+#pragma unroll
+            for (int i = S::win(0) - 1; i > 0; i--)
+                w[i] = w[i - 1];
+            w[0] = xs[POS];
+            levels<0, POS, EVAL>();
+            bin<EVAL, POS + 1>(xs);
+        }
+    }
+
+    // The bin's largest weighted value V, the first level that has it, and whether a weighted
+    // maximum is NaN (an infinite value times a zero weight).
+    __device__ __forceinline__ bool combine(const float (&wt)[S::P], float &V, unsigned int &lev) const
+    {
+        float v[S::P];
+#pragma unroll
+        for (int p = 0; p < S::P; p++)
+            v[p] = wt[p] * mx[p];
+        bool nan = false;
+#pragma unroll
+        for (int p = 0; p < S::P; p += 2)
+            nan |= __builtin_isunordered(v[p], v[(p + 1 < S::P) ? p + 1 : p]);
+        V = v[0];
+        lev = 0;
+        if constexpr (S::P > 1) {
+            V = fmaxf(fmaxf(fmaxf(V, v[1]), v[2]), v[3]);
+#pragma unroll
+            for (int l = 1; l < S::NLEV; l++) {
+                const float u = fmaxf(fmaxf(v[3 * l + 1], v[3 * l + 2]), v[3 * l + 3]);
+                lev = (u > V) ? unsigned(l) : lev;
+                V = fmaxf(V, u);
+            }
+        }
+        return nan;
+    }
+};
+
 __device__ __forceinline__ int pf_level_of_token(unsigned int tok)
 {
     const int p = int((tok >> 8) & 0xffu);
     return (p == 0) ? 0 : (p - 1) / 3;
 }
 
-template<typename Tst, int LW, int LD, bool VAR>
-__global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(VAR ? 2 : PfShape<LW, LD>::WAVES)))
-k_pf(PfArgs a)
+// Rotates a workgroup's rows for the next chunk: positions [Tp, Tp + tpad + flmax) -> [0, ...),
+// i.e. the rows shift down by Tp. Every load of the rows has completed before the caller's last
+// barrier. Done in column blocks of width min(Tp, tpad + flmax) in ascending order, with a
+// barrier between blocks: within a block the positions read ([c0 + Tp, ...)) and
+// written ([c0, c0 + width)) are disjoint, and a later block reads only positions at or
+// above every position an earlier block wrote. Segment 0 rotates; the host chooses
+// segments of at least nwarm*TL + flmax positions, so no other segment reads below
+// tpad + flmax, the positions written here.
+// A thread issues kRot 4-element loads before their stores: element by element, each load waited
+// for the store before it, and segment 0 spent 30-40 memory round trips here.
+template<typename Tst>
+__device__ __forceinline__ void rotate_rows(Tst *rows, int nstreams, const PfArgs &a)
+{
+    constexpr int kRot = 8;
+    const int nrot = a.tpad + a.flmax;
+    const int wcol = min(a.Tp, nrot);            // tpad and Tp are multiples of 4: so is every c0
+    for (int c0 = 0; c0 < nrot; c0 += wcol) {
+        const int nc = min(wcol, nrot - c0), ng = (nc + 3) >> 2;
+        for (int base = 0; base < nstreams * ng; base += kRot * kPfThreads) {
+            rawv_st<Tst, 4> v[kRot];
+#pragma unroll
+            for (int k = 0; k < kRot; k++) {
+                const int idx = min(base + k * kPfThreads + int(threadIdx.x), nstreams * ng - 1);
+                const int s = idx / ng, i = c0 + 4 * (idx - s * ng);
+                v[k] = ldv_raw<Tst, 4>(rows + long(s) * a.rowlen + a.Tp + i);
+            }
+#pragma unroll
+            for (int k = 0; k < kRot; k++) {
+                const int idx = base + k * kPfThreads + int(threadIdx.x);
+                if (idx < nstreams * ng) {
+                    const int s = idx / ng, i = c0 + 4 * (idx - s * ng);
+                    Tst *q = rows + long(s) * a.rowlen + i;
+                    if (i + 4 <= nrot) {
+                        *reinterpret_cast<rawv_st<Tst, 4> *>(q) = v[k];
+                    } else {                      // the row's last samples: no chunk sample past them is written
+                        float e[4];
+                        from_rawv<Tst, 4>(v[k], e);
+#pragma unroll
+                        for (int r = 0; r < 3; r++)
+                            if (i + r < nrot)
+                                st_st_cached(q + r, e[r]);
+                    }
+                }
+            }
+        }
+        if (c0 + wcol < nrot)
+            __syncthreads();
+    }
+}
+
+// With the float64 out_var: every candidate is weighted, compared and summed as it is formed.
+template<typename Tst, int LW, int LD>
+__global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
+k_pf_var(PfArgs a)
 {
     using S = PfShape<LW, LD>;
     constexpr int TL = S::TL, NB = S::NB, STR = TL + 1, VPR = TL / 4;
@@ -267,18 +401,16 @@ k_pf(PfArgs a)
     Tst *outm = reinterpret_cast<Tst *>(a.out_max) + long(b) * a.out_bstride;
     unsigned int *outa = a.out_argmax + long(b) * a.out_bstride;
 
-    PfLane<S, VAR> ln;
+    PfLane<S, true> ln;
 #pragma unroll
     for (int i = 0; i < S::WTOT; i++)
         ln.w[i] = 0.0f;
-    if constexpr (VAR) {
 #pragma unroll
-        for (int p = 0; p < S::P; p++)
-            ln.bs[p] = ln.acc[p] = 0.0;
+    for (int p = 0; p < S::P; p++)
+        ln.bs[p] = ln.acc[p] = 0.0;
 #pragma unroll
-        for (int l = 0; l < S::NLEV; l++)
-            ln.wv[l] = 1.0 / double(a.nt_out * (S::DOUT / S::dt(l)));
-    }
+    for (int l = 0; l < S::NLEV; l++)
+        ln.wv[l] = 1.0 / double(a.nt_out * (S::DOUT / S::dt(l)));
 
     const int nwarm = (a.tpad + TL - 1) / TL;
     const int ntiles = nwarm + ntseg;
@@ -360,37 +492,289 @@ k_pf(PfArgs a)
         }
     }
 
-    if constexpr (VAR) {
-        if (active) {
-            double *ov = a.out_var + long(b) * a.ndm_out * M * S::P + (long(dpf0 + dl) * M + m) * S::P;
+    if (active) {
+        double *ov = a.out_var + long(b) * a.ndm_out * M * S::P + (long(dpf0 + dl) * M + m) * S::P;
 #pragma unroll
-            for (int p = 0; p < S::P; p++)
-                ov[p] = ln.acc[p];
+        for (int p = 0; p < S::P; p++)
+            ov[p] = ln.acc[p];
+    }
+
+    if (blockIdx.z == 0)
+        rotate_rows(rows, nstreams, a);
+}
+
+// The peak finder proper, in two steps. Step 1 walks every stream once and keeps per bin only
+// the largest value of each profile (PfMax: about 1.5 maxima per candidate in place of a
+// multiply, a compare and two selects), weights these, and leaves the stream's largest value
+// and its first level in LDS. Step 2 runs once per kPfBatch bins, one lane per (DM row, bin):
+// it picks the winning multiplet (largest value, then first (level, m)) and walks that one
+// stream over the bin again with PfLane, which gives the value and the token of the first
+// maximum. A DM row has M streams, so step 2 costs 1/M of a full walk per stream.
+// Infinities and NaN: a stream whose windows held one, or whose weighted maxima hold a NaN, is
+// marked, and step 2 walks every stream of a marked (DM row, bin) with PfLane.
+//
+// Samples reach LDS by direct loads (no registers, no conversion), 128 bytes of a row at a
+// time, so that every line is fetched once; a wave stages the 64 rows that its lanes walk, so
+// staging needs no barrier: the next tile's loads start when the wave has read the last part of
+// this one. One load instruction brings 8 rows x 128 bytes; lane i of the
+// instruction writes the i-th 16 bytes, so the 16-byte chunks of a row are permuted on the
+// global side (slot s of row r holds chunk s ^ (r & 7)), and the 16-byte reads of 8
+// neighbouring rows cover all banks. 49 KB of LDS and 168 VGPRs: three workgroups (12 waves)
+// per CU. Bounded by VALU issue (about 400 instructions per stream and 16-sample bin at Wmax 16,
+// against 520 with every candidate compared) and, for float32, near half by the row reads.
+// 16384 DM rows x 2048 samples x 16 beams, Wmax 16, bins of 16: float32 0.774 -> 0.558 ms,
+// float16 0.736 -> 0.444 ms; 36 multiplets, 8 beams of rank 15, float16: 2.28 -> 1.19 ms.
+// Tried: tiles of 16 positions staged through registers (each 128-byte line fetched twice,
+// float32 0.93 ms), two staging buffers and 8 waves per CU (0.68 ms), the walk's float32 loads
+// all at once with bins of 16 (31 registers spilled, 1.31 ms).
+static constexpr int kPfBatch = 12;
+
+typedef __attribute__((address_space(1))) const void *pf_gptr;
+typedef __attribute__((address_space(3))) void *pf_lptr;
+
+template<typename Tst, int LW, int LD>
+__global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(PfShape<LW, LD>::WAVES)))
+k_pf(PfArgs a)
+{
+    using S = PfShape<LW, LD>;
+    constexpr int TL = kPfLine / int(sizeof(Tst));                 // positions per tile
+    constexpr int CH = 16 / int(sizeof(Tst));                      // positions per 16-byte chunk
+    constexpr int SB = (S::DOUT > CH) ? S::DOUT : CH;               // positions read at a time
+    constexpr int BPS = SB / S::DOUT;                               // their bins
+    constexpr int RVS = kPfThreads + 1, RLS = kPfThreads + 4;      // strides of a batch's bins (banks)
+    constexpr int TPAD = (2 * S::W > 4) ? 2 * S::W : 4;             // a.tpad
+    constexpr int NBACK = (TPAD + S::DOUT - 1) / S::DOUT;           // bins that reach into a bin's windows
+    static_assert(TL % SB == 0 && BPS <= kPfBatch, "whole bins per tile");
+    __shared__ __align__(16) unsigned char tile[kPfThreads * kPfLine];
+    __shared__ float rv[kPfBatch * RVS];
+    __shared__ unsigned char rl[kPfBatch * RLS];
+    __shared__ int sn[kPfThreads];               // weight column of each stream
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int M = a.M, N = a.N;
+    const int ndpf = kPfThreads / M;
+    const int dpf0 = blockIdx.x * ndpf;
+    const int b = blockIdx.y;
+    const int ntseg = a.Tp / (TL * a.nseg);      // evaluated tiles of this segment
+    const int tile0 = blockIdx.z * ntseg;        // its first tile in the chunk
+    const int nd = min(ndpf, a.ndm_out - dpf0);
+    const int nstreams = nd * M;
+    const bool active = tid < nstreams;
+    const int dl = tid / M, m = tid - dl * M;
+
+    Tst *rows = reinterpret_cast<Tst *>(a.sb) + long(a.beam0 + b) * a.sb_bstride + long(dpf0) * M * a.rowlen;
+    const int Wds = a.ndm_out / a.ndm_wt;
+    const int Tds = a.nt_out / a.nt_wt;
+    const float *wbeam = a.wt + long(b) * a.wt_bstride;
+    const int wcol = active ? a.m_to_n[m] : 0;
+    const float *wrow = wbeam + long(active ? (dpf0 + dl) / Wds : 0) * a.nt_wt * S::P * N + wcol;
+    sn[tid] = wcol;
+    Tst *outm = reinterpret_cast<Tst *>(a.out_max) + long(b) * a.out_bstride;
+    unsigned int *outa = a.out_argmax + long(b) * a.out_bstride;
+
+    PfMax<S> ln;
+#pragma unroll
+    for (int i = 0; i < S::WTOT; i++)
+        ln.w[i] = 0.0f;
+    int marked = 0;            // bins, from this one on, whose windows hold an infinity or NaN
+
+    // The first tile holds the line of position tpad - 1: nwarm tiles reach back to the line of
+    // position 0 (rows start 'lead' elements after a line; what lies before position 0 in
+    // that line is in the buffer and is older than any window that is evaluated).
+    const int nwarm = (a.tpad + TL - 1) / TL;
+    const int ntiles = nwarm + ntseg;
+    const int srow = 64 * wv + (lane >> 3);                          // row this lane stages, + 8 k
+    const Tst *src = rows + long(srow) * a.rowlen + a.tpad + (tile0 - nwarm) * TL + ((lane & 7) ^ (lane >> 3)) * CH;
+    auto stage = [&](int it) {
+        unsigned char *dst = tile + wv * 64 * kPfLine;
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            if (srow + 8 * k < nstreams)
+                __builtin_amdgcn_global_load_lds((pf_gptr)(src + long(8 * k) * a.rowlen + it * TL),
+                                                 (pf_lptr)(dst + k * 8 * kPfLine), 16, 0, 0);
+    };
+
+    // step 2's DM rows: the wave's own when whole rows fall into a wave, else the workgroup's
+    const bool wave_local = (64 % M) == 0;
+    const int d2 = wave_local ? wv * (64 / M) : 0;
+    const int nd2 = wave_local ? max(0, min(64 / M, nd - d2)) : nd;
+
+    stage(0);
+    int nbatch = 0;            // bins in the batch
+    for (int it = 0; it < ntiles; it++) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // this tile has landed
+        const unsigned char *trow = tile + tid * kPfLine;
+        const int tb0 = (tile0 + it - nwarm) * (TL / S::DOUT);
+#pragma unroll 1
+        for (int sb = 0; sb < TL / SB; sb++) {
+            float x[SB];
+            {
+                rawv_st<Tst, CH> r[SB / CH];
+#pragma unroll
+                for (int c = 0; c < SB / CH; c++)
+                    r[c] = *reinterpret_cast<const rawv_st<Tst, CH> *>(trow + (((sb * (SB / CH) + c) ^ (lane & 7)) << 4));
+#pragma unroll
+                for (int c = 0; c < SB / CH; c++)
+                    from_rawv<Tst, CH>(r[c], x + CH * c);
+            }
+            if (sb + 1 == TL / SB && it + 1 < ntiles) {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's reads of this tile are done
+                stage(it + 1);
+            }
+            if (it < nwarm) {
+#pragma unroll
+                for (int j = 0; j < BPS; j++) {
+                    ln.nonfinite = false;
+                    ln.template bin<false>(x + j * S::DOUT);
+                    marked = ln.nonfinite ? NBACK + 1 : marked;
+                    marked = max(marked - 1, 0);
+                }
+                continue;
+            }
+            const int tbs = tb0 + sb * BPS;
+            if (active) {
+#pragma unroll
+                for (int j = 0; j < BPS; j++) {
+                    // loaded here, used at the end of the bin; kept from bin to bin they would
+                    // be live across step 2, which spills
+                    float wt[S::P];
+                    const float *wp = wrow + long((tbs + j) / Tds) * S::P * N;
+#pragma unroll
+                    for (int p = 0; p < S::P; p++)
+                        wt[p] = wp[p * N];
+                    ln.nonfinite = false;
+                    ln.template bin<true>(x + j * S::DOUT);
+                    float V;
+                    unsigned int lev;
+                    const bool nan = ln.combine(wt, V, lev);
+                    marked = ln.nonfinite ? NBACK + 1 : marked;
+                    rv[(nbatch + j) * RVS + tid] = V;
+                    rl[(nbatch + j) * RLS + tid] = (unsigned char)((marked > 0 || nan) ? 0x80u : lev);
+                    marked = max(marked - 1, 0);
+                }
+            }
+            nbatch += BPS;
+            const bool last = (it + 1 == ntiles && sb + 1 == TL / SB);
+            if (nbatch + BPS <= kPfBatch && !last)
+                continue;
+
+            // ---- step 2 over the batch's bins
+            if (!wave_local)
+                __syncthreads();
+            const int tbb = tbs + BPS - nbatch;
+            for (int idx = wave_local ? lane : tid; idx < nd2 * nbatch; idx += wave_local ? 64 : kPfThreads) {
+                const int d = idx / nbatch + d2, j = idx % nbatch;
+                const float *pv = rv + j * RVS + d * M;
+                const unsigned char *pl = rl + j * RLS + d * M;
+                float V = pv[0];
+                int key = pl[0] * M, m0 = 0;
+                bool all = (pl[0] & 0x80) != 0;
+#pragma unroll 4
+                for (int mm = 1; mm < M; mm++) {
+                    const float v = pv[mm];
+                    const int lv = pl[mm], k = lv * M + mm;
+                    all |= (lv & 0x80) != 0;
+                    if (v > V || (v == V && k < key)) {
+                        V = v;
+                        key = k;
+                        m0 = mm;
+                    }
+                }
+                const int m1 = all ? M : m0 + 1;
+                m0 = all ? 0 : m0;
+
+                const int tb = tbb + j;
+                const float *wp = wbeam + (long((dpf0 + d) / Wds) * a.nt_wt + tb / Tds) * S::P * N;
+                float bv = 0.0f;
+                unsigned int bt = 0;
+                int bk = 0;
+#pragma unroll 1
+                for (int mm = m0; mm < m1; mm++) {
+                    PfLane<S, false> pl2;
+#pragma unroll
+                    for (int i = 0; i < S::WTOT; i++)
+                        pl2.w[i] = 0.0f;
+                    const float *wq = wp + sn[d * M + mm];
+#pragma unroll
+                    for (int p = 0; p < S::P; p++)
+                        pl2.wt[p] = wq[p * N];
+                    const Tst *row = rows + long(d * M + mm) * a.rowlen;
+                    const int pb = a.tpad + tb * S::DOUT;
+                    // groups of V samples; those before position 0 read as zeros (with DOUT >= 4,
+                    // position 0 starts a group)
+                    constexpr int V = (S::DOUT >= 4) ? 4 : 1, NV = S::DOUT / V;
+                    using Raw = typename std::conditional<V == 4, rawv_st<Tst, 4>, raw_st<Tst>>::type;
+                    auto load_bin = [&](Raw (&r)[NV], int pos) {
+#pragma unroll
+                        for (int i = 0; i < NV; i++) {
+                            const Tst *q = row + max(pos + V * i, 0);
+                            if constexpr (V == 4)
+                                r[i] = ldv_raw<Tst, 4>(q);
+                            else
+                                r[i] = ld_raw(q);
+                        }
+                    };
+                    auto floats = [&](const Raw (&r)[NV], int pos, float (&y)[S::DOUT]) {
+#pragma unroll
+                        for (int i = 0; i < NV; i++) {
+                            if constexpr (V == 4)
+                                from_rawv<Tst, 4>(r[i], y + 4 * i);
+                            else
+                                y[i] = from_raw<Tst>(r[i]);
+#pragma unroll
+                            for (int q = 0; q < V; q++)
+                                y[V * i + q] = (pos + V * i >= 0) ? y[V * i + q] : 0.0f;
+                        }
+                    };
+                    float y[S::DOUT];
+                    if constexpr ((NBACK + 1) * S::DOUT <= (sizeof(Tst) == 2 ? 64 : 40) && NBACK <= 8) {
+                        // all of the walk's loads at once
+                        Raw r[NBACK + 1][NV];
+#pragma unroll
+                        for (int k = 0; k <= NBACK; k++)
+                            load_bin(r[k], pb + (k - NBACK) * S::DOUT);
+#pragma unroll
+                        for (int k = 0; k < NBACK; k++) {
+                            floats(r[k], pb + (k - NBACK) * S::DOUT, y);
+                            pl2.template bin<false>(y);
+                        }
+                        floats(r[NBACK], pb, y);
+                    } else {
+                        Raw r[NV];
+#pragma unroll 1
+                        for (int k = NBACK; k > 0; k--) {
+                            load_bin(r, pb - k * S::DOUT);
+                            floats(r, pb - k * S::DOUT, y);
+                            pl2.template bin<false>(y);
+                        }
+                        load_bin(r, pb);
+                        floats(r, pb, y);
+                    }
+                    pl2.template bin<true>(y);
+                    float v;
+                    unsigned int c;
+                    pl2.combine(v, c);
+                    const int k = pf_level_of_token(c) * M + mm;
+                    if (mm == m0 || v > bv || (v == bv && k < bk)) {
+                        bv = v;
+                        bt = c | (unsigned(mm) << 16);
+                        bk = k;
+                    }
+                }
+                const long o = long(dpf0 + d) * a.nt_out + tb;
+                st_st(outm + o, bv);
+                outa[o] = bt;
+            }
+            nbatch = 0;
+            if (!wave_local)
+                __syncthreads();       // rv and rl are free
         }
     }
 
-    // ---- rotate rows for the next chunk: positions [Tp, Tp + tpad + flmax) -> [0, ...),
-    // i.e. the rows shift down by Tp. All staging loads completed before the last barrier.
-    // Done in column blocks of width min(Tp, tpad + flmax) in ascending order, with a
-    // barrier between blocks: within a block the positions read ([c0 + Tp, ...)) and
-    // written ([c0, c0 + width)) are disjoint, and a later block reads only positions at or
-    // above every position an earlier block wrote. Segment 0 rotates; the host chooses
-    // segments of at least nwarm*TL + flmax positions, so no other segment reads below
-    // tpad + flmax, the positions written here.
-    if (blockIdx.z != 0)
-        return;
-    const int nrot = a.tpad + a.flmax;
-    const int wcol = min(a.Tp, nrot);
-    for (int c0 = 0; c0 < nrot; c0 += wcol) {
-        const int nc = min(wcol, nrot - c0);
-        for (int idx = tid; idx < nstreams * nc; idx += kPfThreads) {
-            const int s = idx / nc, i = c0 + (idx - s * nc);
-            Tst *row = rows + long(s) * a.rowlen;
-            const Tst v = row[a.Tp + i];
-            row[i] = v;
-        }
-        if (c0 + wcol < nrot)
-            __syncthreads();
+    if (blockIdx.z == 0) {
+        __syncthreads();               // step 2 has read the rows
+        rotate_rows(rows, nstreams, a);
     }
 }
 
@@ -402,9 +786,9 @@ static void launch_pf_lw(const PfArgs &a, hipStream_t st, dim3 grid)
 #define PDD_PF(LDV)                                                                \
         case (1 << LDV):                                                           \
             if (a.out_var)                                                         \
-                hipLaunchKernelGGL((k_pf<Tst, LW, LDV, true>), grid, block, 0, st, a);  \
+                hipLaunchKernelGGL((k_pf_var<Tst, LW, LDV>), grid, block, 0, st, a);  \
             else                                                                   \
-                hipLaunchKernelGGL((k_pf<Tst, LW, LDV, false>), grid, block, 0, st, a); \
+                hipLaunchKernelGGL((k_pf<Tst, LW, LDV>), grid, block, 0, st, a); \
             break;
         PDD_PF(0) PDD_PF(1) PDD_PF(2) PDD_PF(3) PDD_PF(4) PDD_PF(5)
 #undef PDD_PF
@@ -415,11 +799,10 @@ static void launch_pf_lw(const PfArgs &a, hipStream_t st, dim3 grid)
 // Time segments per chunk: the fewest (a power of two) that give at least a.target_blocks
 // workgroups (2048 unless tuned), within segments of whole tiles of at least
 // nwarm*TL + flmax positions (see the rotation in k_pf). With out_var, one segment.
-static int pf_nseg(const PfArgs &a, long nblocks)
+static int pf_nseg(const PfArgs &a, long nblocks, int TL)
 {
     if (a.out_var)
         return 1;
-    const int TL = pf_tile_len(a.Dout);
     const int nwarm = (a.tpad + TL - 1) / TL;
     int nseg = 1;
     while (nblocks * nseg < a.target_blocks) {
@@ -437,7 +820,7 @@ static void launch_pf_t(const PfArgs &a0, hipStream_t st)
     PfArgs a = a0;
     const int ndpf = kPfThreads / a.M;
     const unsigned nbx = unsigned((a.ndm_out + ndpf - 1) / ndpf);
-    a.nseg = pf_nseg(a, long(nbx) * a.B);
+    a.nseg = pf_nseg(a, long(nbx) * a.B, kPfLine / int(sizeof(Tst)));
     dim3 grid{nbx, unsigned(a.B), unsigned(a.nseg)};
     switch ((a.P - 1) / 3) {
         case 0: launch_pf_lw<Tst, 0>(a, st, grid); break;
