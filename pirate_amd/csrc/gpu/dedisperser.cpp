@@ -16,9 +16,7 @@ namespace pirate_amd {
             throw pdd_error(std::string("HIP error: ") + hipGetErrorString(_e) + " in " + #expr); \
     } while (0)
 
-static constexpr int kGpuMaxDD = 8;          // register-tree kernels (stage 1, final-pass stage 2)
-static constexpr int kGpuMaxDDGeneral = 7;   // LDS-tile stage 2 (subband searches)
-static constexpr long kLdsBytesPerCU = 160 * 1024;
+static constexpr int kGpuMaxDD = 8;          // tree kernels, per stage
 
 
 GpuDedisperser::GpuDedisperser(std::shared_ptr<DedispersionPlan> plan_, const GpuDedisperserParams &params_) :
@@ -81,15 +79,13 @@ GpuDedisperser::~GpuDedisperser()
         if (h)
             (void) hipHostFree(h);
     for (auto *v : {&rings, &ring_row_off, &ring_row_cap, &ring1_row_off, &ring1_row_cap, &spill_rows,
-                    &stage2_lags, &sb, &d_main_emit, &d_stag,
-                    &d_lvl0, &d_fl, &d_m_to_n, &d_stag_begin, &d_stag_goff, &d_out_stream, &s1_state, &s2_state, &weights, &out_var})
+                    &stage2_lags, &sb, &d_m_to_n, &s1_state, &s2_state, &weights, &out_var})
         for (auto &a : *v)
             freeit(a);
     freeit(scorer_params);
     freeit(scorer_origins);
     freeit(scorer_out);
     freeit(out_region);     // out_max / out_argmax are views into it
-    freeit(split_x);
     for (auto &t : timed_pending) {
         timing_event_pool.push_back(t.start);
         timing_event_pool.push_back(t.stop);
@@ -101,8 +97,6 @@ GpuDedisperser::~GpuDedisperser()
         for (size_t p = 1; p < bs.size(); p++)
             if (bs[p])
                 (void) hipStreamDestroy(bs[p]);
-    if (ev_split_free)
-        (void) hipEventDestroy(ev_split_free);
     for (auto &v : ev_join)
         for (hipEvent_t e : v)
             (void) hipEventDestroy(e);
@@ -115,11 +109,8 @@ GpuDedisperser::~GpuDedisperser()
 }
 
 
-// Subband-stream tables of each stage-2 tree. The loops restate the subband extraction
-// of ReferenceTree::dedisperse_2d (src_lib/ReferenceTree.cpp:142-287) for one tree
-// instance: level-0 copies, main-pair outputs (even subband index), staggered extra
-// butterflies (odd subband index), multiplet numbering, and the final lags
-// (ReferenceTree.cpp:42-54).
+// Subband bands of each stage-2 tree (multiplet numbering of FrequencySubbands, level by level)
+// and the shape of its peak-finder rows.
 void GpuDedisperser::build_tables()
 {
     tables.resize(ntrees);
@@ -127,112 +118,23 @@ void GpuDedisperser::build_tables()
         const DedispersionTree &t = plan->trees[it];
         const FrequencySubbands &fs = t.frequency_subbands;
         TreeTables &T = tables[it];
-        const int dd = t.dd_rank, pf_rank = int(fs.pf_rank);
-        const int NP = 1 << (dd - 1), M = int(fs.M);
-        const int pf_ndm = 1 << (dd - pf_rank);
-        T.M = M;
+        const int pf_rank = int(fs.pf_rank);
+        PDD_CHECK(pf_rank == (t.dd_rank + 1) / 2 && pf_rank <= kMaxPfRank,
+                  "GpuDedisperser: internal error: unexpected peak-finding rank");
+        T.M = int(fs.M);
         T.N = int(fs.N);
-        T.main_emit.assign(dd * NP, -1);
-        T.fl.assign(pf_ndm * M, 0);
-        long mcurr = 0;
-        int hoff = 0;
-        for (int r = 0; r <= dd; r++) {
-            const int ndm_in = 1 << r;
-            if (r == dd - pf_rank) {
-                const int pf_ns = int(fs.subband_counts[0]);
-                for (int dm_in = 0; dm_in < ndm_in; dm_in++)
-                    for (int pfs = 0; pfs < pf_ns; pfs++) {
-                        T.lvl0.push_back(pfs * ndm_in + int(bit_reverse(dm_in, r)));
-                        T.lvl0.push_back(dm_in * M + pfs);
-                    }
-                mcurr += pf_ns;
-            }
-            if (r >= dd)
-                break;
-            const int pf_level = r + pf_rank - dd + 1;
-            if (pf_level <= 0)
-                continue;
-            const int pf_ns = int(fs.subband_counts[pf_level]);
-            const int pf_nd2 = 1 << (pf_level - 1);
-            for (int pf_dm = 0; pf_dm < pf_ndm; pf_dm++)
-                for (int d2 = 0; d2 < pf_nd2; d2++) {
-                    const int dm_in = pf_dm * pf_nd2 + d2;
-                    const int dmb = int(bit_reverse(dm_in, r));
-                    for (int pfs = 0; pfs < pf_ns; pfs++) {
-                        const int m = int(mcurr) + pfs * 2 * pf_nd2 + 2 * d2;
-                        const int s0 = pf_dm * M + m;
-                        if ((pfs & 1) == 0) {
-                            const int p = (pfs / 2) * ndm_in + dmb;
-                            T.main_emit[r * NP + p] = s0;
-                        }
-                        else {
-                            int e[6] = {r, pfs * ndm_in + dmb, (pfs + 1) * ndm_in + dmb, dm_in, s0, hoff};
-                            T.stag.insert(T.stag.end(), e, e + 6);
-                            hoff += ndm_in;
-                        }
-                    }
-                }
-            mcurr += long(pf_ns) * 2 * pf_nd2;
+        int m = 0;
+        for (int lev = 0; lev <= pf_rank; lev++) {
+            T.nband.push_back(int(fs.subband_counts[lev]));
+            T.mband.push_back(m);
+            m += T.nband[lev] << lev;
         }
-        PDD_CHECK(mcurr == M, "GpuDedisperser: internal error: multiplet count mismatch");
-        T.nstag = int(T.stag.size() / 6);
-        // Entries were generated pass by pass: record each pass's range.
-        T.stag_begin.assign(dd + 1, 0);
-        for (int r = 0, k = 0; r <= dd; r++) {
-            while (k < T.nstag && T.stag[6 * k] < r)
-                k++;
-            T.stag_begin[r] = k;
+        PDD_CHECK(m == T.M, "GpuDedisperser: internal error: multiplet count mismatch");
+        // largest final lag of a stream (ReferenceTree.cpp:42-54)
+        for (int k = 0; k < T.M; k++) {
+            T.flmax = std::max(T.flmax, int((pow2(pf_rank) - fs.m_to_fhi(k)) * (pow2(t.dd_rank - pf_rank) - 1)));
+            T.m_to_n.push_back(int(fs.m_to_n[k]));
         }
-        T.nlvl0 = int(T.lvl0.size() / 2);
-        T.stag_hist_nelts = hoff;
-        if (dd == 8) {
-            // Rank-8 split: each group of rows with equal low 4 bits keeps only the histories
-            // of its own staggered pairs (group = row0 & 15), packed.
-            std::vector<int> gtot(16, 0);
-            T.stag_goff.assign(T.nstag, 0);
-            for (int k = 0; k < T.nstag; k++) {
-                const int g = T.stag[6 * k + 1] & 15;
-                T.stag_goff[k] = gtot[g];
-                gtot[g] += 1 << T.stag[6 * k];
-            }
-            T.stag_hist_g = *std::max_element(gtot.begin(), gtot.end());
-        }
-
-        // Register-tree path: every stream is a final-pass output (main pairs of the last
-        // pass, or level-0 copies after the last pass), each row feeding at most one stream.
-        T.out_stream.assign(pow2(dd), -1);
-        T.fast = (T.nstag == 0);
-        for (int r = 0; r < dd && T.fast; r++)
-            for (int p = 0; p < NP; p++) {
-                const int s0 = T.main_emit[r * NP + p];
-                if (s0 < 0)
-                    continue;
-                if (r != dd - 1 || T.out_stream[p] >= 0 || T.out_stream[p + NP] >= 0)
-                    T.fast = false;
-                else {
-                    T.out_stream[p] = s0;
-                    T.out_stream[p + NP] = s0 + 1;
-                }
-            }
-        if (T.nlvl0 > 0 && dd - pf_rank != dd)
-            T.fast = false;
-        for (int k = 0; k < T.nlvl0 && T.fast; k++) {
-            const int row = T.lvl0[2 * k], s0 = T.lvl0[2 * k + 1];
-            if (T.out_stream[row] >= 0)
-                T.fast = false;
-            else
-                T.out_stream[row] = s0;
-        }
-        T.split = !T.fast && dd == 8;
-
-        for (int pf_dm = 0; pf_dm < pf_ndm; pf_dm++)
-            for (int m = 0; m < M; m++) {
-                int v = int((pow2(pf_rank) - fs.m_to_fhi(m)) * pf_dm);
-                T.fl[pf_dm * M + m] = v;
-                T.flmax = std::max(T.flmax, v);
-            }
-        for (int m = 0; m < M; m++)
-            T.m_to_n.push_back(int(fs.m_to_n[m]));
 
         T.tpad = int(std::max(2 * t.pf.max_width, 4L));
         T.nlev = std::max(integer_log2(t.pf.max_width), 1);
@@ -241,7 +143,7 @@ void GpuDedisperser::build_tables()
         // and the peak finder's loads then cover whole lines.
         const int line_elts = int(128 / elt_bytes);
         T.lead = int(align_up(T.tpad, line_elts)) - T.tpad;
-        T.rowlen = int(align_up(T.tpad + t.nt_ds + T.flmax, line_elts));
+        T.rowlen = int(align_up(T.tpad + t.nt_ds, line_elts));
     }
 }
 
@@ -268,14 +170,6 @@ void GpuDedisperser::validate_gpu_limits()
         const DedispersionTree &t = plan->trees[it];
         const TreeTables &T = tables[it];
         PDD_CHECK(t.dd_rank <= kGpuMaxDD, "GpuDedisperser: stage-2 dd_rank " << t.dd_rank << " not supported by pirate_amd (max " << kGpuMaxDD << ")");
-        if (!T.fast && t.dd_rank <= kGpuMaxDDGeneral)
-            PDD_CHECK(stage2_lds_bytes(t.dd_rank, T.stag_hist_nelts) <= kLdsBytesPerCU,
-                      "GpuDedisperser: tree " << it << " needs too much LDS (subband history)");
-        if (!T.fast && t.dd_rank == 8) {
-            PDD_CHECK(t.frequency_subbands.pf_rank <= 4, "GpuDedisperser: tree " << it << ": rank-8 split needs pf_rank <= 4");
-            PDD_CHECK(split_b_lds_bytes(T.stag_hist_g) <= kLdsBytesPerCU,
-                      "GpuDedisperser: tree " << it << " needs too much LDS (subband history)");
-        }
         PDD_CHECK(t.pf.time_downsampling <= 512, "GpuDedisperser: time_downsampling too large");
         PDD_CHECK(pf_config_supported(T.M, T.tpad, T.nlev, int(t.Dcore), int(t.pf.time_downsampling), t.nt_ds),
                   "GpuDedisperser: tree " << it << ": peak-finder shape not supported (M=" << T.M << ")");
@@ -447,21 +341,13 @@ void GpuDedisperser::allocate()
             std::memset(host_ring[p], 0, hb);
             host_bytes_allocated += hb;
         }
-        s1_state_bstride[p] = pow2(amb1) * fast_tree_state_nelts(int(dd1));
+        s1_state_bstride[p] = 2 * pow2(amb1) * tree_state_nelts(int(dd1));      // two chunk parities
         s1_state[p] = dalloc(size_t(total_beams) * s1_state_bstride[p] * sizeof(float));
     }
 
-    size_t split_nelts = 0;   // float32 scratch of rank-8 split stage-2 trees
     stage2_lags.resize(ntrees);
     sb.resize(ntrees);
-    d_main_emit.resize(ntrees);
-    d_stag.resize(ntrees);
-    d_lvl0.resize(ntrees);
-    d_fl.resize(ntrees);
     d_m_to_n.resize(ntrees);
-    d_stag_begin.resize(ntrees);
-    d_stag_goff.resize(ntrees);
-    d_out_stream.resize(ntrees);
     s2_state.resize(ntrees);
     s2_state_bstride.resize(ntrees);
     weights.resize(ntrees);
@@ -479,24 +365,12 @@ void GpuDedisperser::allocate()
                 lags[rr] = int(rb_lag(fc, j, t.amb_rank, t.dd_rank, t.primary_tree_index > 0) - kr[rr] * t.nt_ds);
             }
         stage2_lags[it] = up_int(lags);
-        // Peak-finder input rows hold per-beam history (and final-lag "future" samples)
-        // across chunks: one set of rows per beam of the GPU, not per batch.
+        // Peak-finder input rows hold per-beam history across chunks: one set of rows per beam of the GPU, not per batch.
         PDD_CHECK(t.ndm_out * T.M * T.rowlen < (1L << 31), "GpuDedisperser: peak-finder rows of tree " << it
                   << " exceed 2^31 elements per beam");
         sb[it] = dalloc((size_t(total_beams) * t.ndm_out * T.M * T.rowlen + T.lead) * elt_bytes);
-        d_main_emit[it] = up_int(T.main_emit);
-        d_stag[it] = up_int(T.stag);
-        d_lvl0[it] = up_int(T.lvl0);
-        d_fl[it] = up_int(T.fl);
         d_m_to_n[it] = up_int(T.m_to_n);
-        d_stag_begin[it] = up_int(T.stag_begin);
-        d_stag_goff[it] = up_int(T.stag_goff);
-        d_out_stream[it] = up_int(T.out_stream);
-        s2_state_bstride[it] = pow2(t.amb_rank) * (T.fast ? fast_tree_state_nelts(t.dd_rank)
-                                                   : T.split ? split_state_nelts_per_tree(T.stag_hist_g)
-                                                             : stage2_state_nelts_per_tree(t.dd_rank, T.stag_hist_nelts));
-        if (T.split)
-            split_nelts = std::max(split_nelts, size_t(B) * pow2(t.amb_rank) * 256 * t.nt_ds);
+        s2_state_bstride[it] = 2 * pow2(t.amb_rank) * tree_state_nelts(t.dd_rank);      // two chunk parities
         s2_state[it] = dalloc(size_t(total_beams) * s2_state_bstride[it] * sizeof(float));
         weights[it] = dalloc(size_t(nbatches_wt) * B * t.ndm_wt * t.nt_wt * t.nprofiles * T.N * sizeof(float));
         // out_max / out_argmax: views into the output region (below)
@@ -505,9 +379,6 @@ void GpuDedisperser::allocate()
         if (params.enable_variances)
             out_var[it] = dalloc(size_t(nbatches_out) * B * t.ndm_out * T.M * t.nprofiles * sizeof(double));
     }
-
-    if (split_nelts > 0)
-        split_x = dalloc(split_nelts * sizeof(float));
 
     // Output ring: every tree's out_max and out_argmax in one device allocation (256-byte
     // aligned sub-arrays, tree-major), so that one IPC handle exports all of it to a
@@ -551,7 +422,6 @@ void GpuDedisperser::allocate()
     }
     mkev(ev_fork, nstreams);
     mkev(ev_batch_done, nbatches);
-    HIP_CHECK(hipEventCreateWithFlags(&ev_split_free, hipEventDisableTiming));
     mkev(ev_input_free, nstreams);
     mkev(ev_input_ready, nstreams);
     mkev(ev_output_ready, nbatches_out);
@@ -673,15 +543,16 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
         if (nspill[p] > 0)
             spill_h2d(p, ichunk, ibatch, beam0);
     // Primary tree p's stage 1, spill scatter, stage-2 trees and peak finders run on branch
-    // stream p (0: st); st waits for every branch at the end. The branches p >= 1 start
-    // after the gridding, or, when tree 0's stage 2 is the register-tree kernel, after it:
-    // stage 1 and that stage 2 run near the HBM bandwidth on their own (chord16k fp32:
-    // 5.57 ms/step serial, 5.66 with the branches from the gridding on), while the
-    // peak finders and the subband stage-2 kernels are bound by VALU or LDS latency and
-    // leave bandwidth to share (chime_sb1-shaped, fp16: 15.68 -> 15.11 ms).
+    // stream p (0: st); st waits for every branch at the end. The branches p >= 1 start after tree
+    // 0's stage 2 when its instances alone fill the chip, else right after the gridding: stage 1
+    // and stage 2 of tree 0 then run near the HBM bandwidth on their own, and what the branches
+    // share best is the peak finder's time (16 beams x 16384 channels: late 5.44 ms, early
+    // 5.49 ms; float16 4.06 and 4.16 ms; rank 15 with subbands 5.32 and 5.58 ms). Small chains
+    // only gain from kernels side by side (2 beams of rank 8, 3 primary trees: 0.37 and 0.32 ms).
     // tuning.fork == 2: every branch on 'st' in order (one kernel at a time, for per-kernel timing).
     const bool serial = (tuning.fork == 2);
-    const bool late_fork = (tuning.fork < 0) ? tables[0].fast : (tuning.fork == 1);
+    const bool full = (B << plan->stage1_dd_rank[0]) >= 256;      // stage-2 instances of tree 0, one per CU
+    const bool late_fork = (tuning.fork < 0) ? full : (tuning.fork == 1);
     if (!late_fork && !serial)
         HIP_CHECK(hipEventRecord(ev_fork_s, st));
     for (long p = 0; p < npri; p++) {
@@ -710,7 +581,7 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
         timed_begin(nm, sp, ev);
         if (nspill[p] > 0)     // the outbox is free once the previous chunk's copy has read it
             HIP_CHECK(hipStreamWaitEvent(sp, ev_spill_d2h[p * nbatches + ibatch], 0));
-        launch_stage1_fast(dtype, s, sp);
+        launch_stage1(dtype, s, sp);
         timed_end(nm, sp, ev);
         if (nspill[p] > 0) {
             spill_d2h(p, ichunk, ibatch, beam0, sp);
@@ -731,17 +602,11 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
             s2.sb_bstride = t.ndm_out * T.M * T.rowlen;
             s2.rowlen = T.rowlen;
             s2.tpad = T.tpad;
-            s2.main_emit = (const int *) d_main_emit[it].ptr;
-            s2.stag = (const int *) d_stag[it].ptr;
-            s2.lvl0 = (const int *) d_lvl0[it].ptr;
-            s2.fl = (const int *) d_fl[it].ptr;
-            s2.nstag = T.nstag;
-            s2.nlvl0 = T.nlvl0;
-            s2.stag_hist_nelts = T.split ? T.stag_hist_g : T.stag_hist_nelts;
-            s2.stag_goff = (const int *) d_stag_goff[it].ptr;
-            s2.stag_begin = (const int *) d_stag_begin[it].ptr;
             s2.M = T.M;
-            s2.pf_rank = int(t.frequency_subbands.pf_rank);
+            for (size_t lev = 0; lev <= kMaxPfRank; lev++) {
+                s2.nband[lev] = (lev < T.nband.size()) ? T.nband[lev] : 0;
+                s2.mband[lev] = (lev < T.mband.size()) ? T.mband[lev] : 0;
+            }
             s2.state = (float *) s2_state[it].ptr;
             s2.state_bstride = s2_state_bstride[it];
             s2.B = int(B);
@@ -749,23 +614,12 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
             s2.dd = t.dd_rank;
             s2.Tp = t.nt_ds;
             s2.beam0 = beam0;
-            s2.amb1_dd1 = t.amb_rank;
             s2.chunk = ichunk;
             s2.chunk_dev = chunk_dev;
-            s2.out_stream = (const int *) d_out_stream[it].ptr;
             hipEvent_t ev2;
             const std::string nm2 = "stage2_t" + std::to_string(it);
             timed_begin(nm2, sp, ev2);
-            if (T.fast)
-                launch_stage2_fast(dtype, s2, sp);
-            else if (T.split) {
-                // the float32 scratch is shared by every rank-8 split tree
-                HIP_CHECK(hipStreamWaitEvent(sp, ev_split_free, 0));
-                launch_stage2_split(dtype, s2, (float *) split_x.ptr, sp);
-                HIP_CHECK(hipEventRecord(ev_split_free, sp));
-            }
-            else
-                launch_stage2(dtype, s2, sp);
+            launch_stage2(dtype, s2, sp);
             timed_end(nm2, sp, ev2);
             if (late_fork && !serial && it == 0)
                 HIP_CHECK(hipEventRecord(ev_fork_s, st));
@@ -795,7 +649,6 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
             f.sb_bstride = s2.sb_bstride;
             f.rowlen = T.rowlen;
             f.tpad = T.tpad;
-            f.flmax = T.flmax;
             f.m_to_n = (const int *) d_m_to_n[it].ptr;
             const long wslot_n = B * t.ndm_wt * t.nt_wt * t.nprofiles * T.N;
             f.wt = (const float *) weights[it].ptr + wslot * wslot_n;

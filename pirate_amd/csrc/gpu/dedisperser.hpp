@@ -158,16 +158,13 @@ public:
     // returns, so that the primary trees' kernels overlap.
     std::vector<std::vector<hipStream_t>> branch_streams;
 
-    // Per-tree stage-2 tables (host copies, exposed for tests).
+    // Per-tree stage-2 and peak-finder shapes.
     struct TreeTables {
-        std::vector<int> main_emit, stag, lvl0, fl, m_to_n, stag_begin;
-        std::vector<int> out_stream;   // register-tree path: final row -> stream (-1: none)
-        bool fast = false;             // stage 2 runs on the register-tree kernel
-        bool split = false;            // rank-8 subband search: two-launch split kernel
-        int nstag = 0, nlvl0 = 0, stag_hist_nelts = 0, flmax = 0, tpad = 0, nlev = 0, rowlen = 0, M = 0, N = 0;
+        std::vector<int> m_to_n;
+        std::vector<int> nband, mband; // subband bands and first multiplet per level 0..pf_rank
+        int flmax = 0;                 // largest subband final lag
+        int tpad = 0, nlev = 0, rowlen = 0, M = 0, N = 0;
         int lead = 0;                  // element offset of the peak-finder rows in their buffer
-        std::vector<int> stag_goff;    // rank 8: staggered history offset within its row group
-        int stag_hist_g = 0;           // rank 8: staggered history floats per row group
     };
     std::vector<TreeTables> tables;
 
@@ -202,7 +199,6 @@ private:
     std::vector<long> nspill, outbox_off, inbox_off, host_bstride;   // [p]
     hipStream_t d2h_stream = nullptr, h2d_stream = nullptr;
     std::vector<hipEvent_t> ev_spill_s1, ev_spill_d2h, ev_spill_h2d, ev_spill_scatter;   // [p * nbatches + batch]
-    hipEvent_t ev_split_free = nullptr;
     std::vector<hipEvent_t> ev_fork;                          // [s]
     std::vector<std::vector<hipEvent_t>> ev_join;             // [s][p]
     std::vector<hipEvent_t> ev_batch_done;                    // [batch]: latest chain of the batch
@@ -211,14 +207,13 @@ private:
     std::vector<void *> host_ring;                           // [p] pinned, (total_beams, host_bstride)
     std::vector<DeviceArray> stage2_lags;    // [itree] device int
     std::vector<DeviceArray> sb;      // [itree] (B, ndm_out, M, rowlen)
-    std::vector<DeviceArray> d_main_emit, d_stag, d_lvl0, d_fl, d_m_to_n, d_stag_begin, d_stag_goff, d_out_stream;
+    std::vector<DeviceArray> d_m_to_n;
     DeviceArray lds_state;  long lds_state_bstride = 0;
     std::vector<DeviceArray> s1_state; std::vector<long> s1_state_bstride;
     std::vector<DeviceArray> s2_state; std::vector<long> s2_state_bstride;
     std::vector<DeviceArray> weights; // [itree] (nbatches_wt, B, ndm_wt, nt_wt, P, N) float
     std::vector<DeviceArray> out_max, out_argmax;   // [itree] (nbatches_out, B, ndm_out, nt_out), views into out_region
     DeviceArray out_region;
-    DeviceArray split_x;              // float32 scratch of the rank-8 split stage 2
     std::vector<size_t> out_offsets;                // [2 * itree + which]
     std::vector<DeviceArray> out_var; // [itree] (nbatches_out, B, ndm_out, M, P) float64, if enabled
     // learned scorer (set_scorer): tree, parameters, tile origins of one batch, logits ring

@@ -102,9 +102,23 @@ __device__ __forceinline__ void st_st(__hip_bfloat16 *p, float x)
     __builtin_nontemporal_store(st_bits(p, x), reinterpret_cast<unsigned short *>(p));
 }
 
+typedef float f32x2_nt __attribute__((ext_vector_type(2)));
 typedef float f32x4_nt __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2_nt __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4_nt __attribute__((ext_vector_type(4)));
+
+// Two consecutive storage elements from float, at an even element offset (nontemporal).
+__device__ __forceinline__ void st2_st(float *p, float x, float y)
+{
+    const f32x2_nt t = {x, y};
+    __builtin_nontemporal_store(t, reinterpret_cast<f32x2_nt *>(p));
+}
+
+template<typename T16>
+__device__ __forceinline__ void st2_st(T16 *p, float x, float y)
+{
+    __builtin_nontemporal_store(unsigned(st_bits(p, x)) | (unsigned(st_bits(p, y)) << 16), reinterpret_cast<unsigned *>(p));
+}
 
 // Four consecutive storage elements from float (round-to-nearest-even for 16-bit types),
 // to global memory (nontemporal).

@@ -27,8 +27,8 @@
 // candidate, equal those of one lane walking the whole chunk. The running variance sums
 // depend on the order of the bins, so they use one segment.
 //
-// Rows are [tpad history | Tp samples | future (final lags)]; at the end of a chunk the
-// history and future regions are rotated into place for the next chunk.
+// Rows are [tpad history | Tp samples]; at the end of a chunk the last tpad samples are moved to
+// the front for the next chunk.
 
 #include "device_common.hpp"
 #include "kernels.hpp"
@@ -320,52 +320,39 @@ __device__ __forceinline__ int pf_level_of_token(unsigned int tok)
     return (p == 0) ? 0 : (p - 1) / 3;
 }
 
-// Rotates a workgroup's rows for the next chunk: positions [Tp, Tp + tpad + flmax) -> [0, ...),
-// i.e. the rows shift down by Tp. Every load of the rows has completed before the caller's last
-// barrier. Done in column blocks of width min(Tp, tpad + flmax) in ascending order, with a
+// Rotates a workgroup's rows for the next chunk: positions [Tp, Tp + tpad) -> [0, tpad), i.e.
+// the rows shift down by Tp. Every load of the rows has completed before the caller's last
+// barrier. Done in column blocks of width min(Tp, tpad) in ascending order, with a
 // barrier between blocks: within a block the positions read ([c0 + Tp, ...)) and
 // written ([c0, c0 + width)) are disjoint, and a later block reads only positions at or
 // above every position an earlier block wrote. Segment 0 rotates; the host chooses
-// segments of at least nwarm*TL + flmax positions, so no other segment reads below
-// tpad + flmax, the positions written here.
-// A thread issues kRot 4-element loads before their stores: element by element, each load waited
-// for the store before it, and segment 0 spent 30-40 memory round trips here.
+// segments of at least nwarm*TL positions, so no other segment reads below tpad, the positions
+// written here. A thread issues kRot 4-element loads before their stores: element by element,
+// each load waited for the store before it, and segment 0 spent 30-40 memory round trips here.
 template<typename Tst>
 __device__ __forceinline__ void rotate_rows(Tst *rows, int nstreams, const PfArgs &a)
 {
     constexpr int kRot = 8;
-    const int nrot = a.tpad + a.flmax;
-    const int wcol = min(a.Tp, nrot);            // tpad and Tp are multiples of 4: so is every c0
-    for (int c0 = 0; c0 < nrot; c0 += wcol) {
-        const int nc = min(wcol, nrot - c0), ng = (nc + 3) >> 2;
-        for (int base = 0; base < nstreams * ng; base += kRot * kPfThreads) {
+    const int wcol = min(a.Tp, a.tpad);          // tpad and Tp are multiples of 4: so is every c0
+    for (int c0 = 0; c0 < a.tpad; c0 += wcol) {
+        const int ng = min(wcol, a.tpad - c0) >> 2, n = nstreams * ng;
+        for (int base = 0; base < n; base += kRot * kPfThreads) {
             rawv_st<Tst, 4> v[kRot];
 #pragma unroll
             for (int k = 0; k < kRot; k++) {
-                const int idx = min(base + k * kPfThreads + int(threadIdx.x), nstreams * ng - 1);
+                const int idx = min(base + k * kPfThreads + int(threadIdx.x), n - 1);
                 const int s = idx / ng, i = c0 + 4 * (idx - s * ng);
                 v[k] = ldv_raw<Tst, 4>(rows + long(s) * a.rowlen + a.Tp + i);
             }
 #pragma unroll
             for (int k = 0; k < kRot; k++) {
                 const int idx = base + k * kPfThreads + int(threadIdx.x);
-                if (idx < nstreams * ng) {
-                    const int s = idx / ng, i = c0 + 4 * (idx - s * ng);
-                    Tst *q = rows + long(s) * a.rowlen + i;
-                    if (i + 4 <= nrot) {
-                        *reinterpret_cast<rawv_st<Tst, 4> *>(q) = v[k];
-                    } else {                      // the row's last samples: no chunk sample past them is written
-                        float e[4];
-                        from_rawv<Tst, 4>(v[k], e);
-#pragma unroll
-                        for (int r = 0; r < 3; r++)
-                            if (i + r < nrot)
-                                st_st_cached(q + r, e[r]);
-                    }
-                }
+                const int s = idx / ng, i = c0 + 4 * (idx - s * ng);
+                if (idx < n)
+                    *reinterpret_cast<rawv_st<Tst, 4> *>(rows + long(s) * a.rowlen + i) = v[k];
             }
         }
-        if (c0 + wcol < nrot)
+        if (c0 + wcol < a.tpad)
             __syncthreads();
     }
 }
@@ -798,7 +785,7 @@ static void launch_pf_lw(const PfArgs &a, hipStream_t st, dim3 grid)
 
 // Time segments per chunk: the fewest (a power of two) that give at least a.target_blocks
 // workgroups (2048 unless tuned), within segments of whole tiles of at least
-// nwarm*TL + flmax positions (see the rotation in k_pf). With out_var, one segment.
+// nwarm*TL positions (see rotate_rows). With out_var, one segment.
 static int pf_nseg(const PfArgs &a, long nblocks, int TL)
 {
     if (a.out_var)
@@ -807,7 +794,7 @@ static int pf_nseg(const PfArgs &a, long nblocks, int TL)
     int nseg = 1;
     while (nblocks * nseg < a.target_blocks) {
         const int n2 = 2 * nseg;
-        if (a.Tp % (TL * n2) != 0 || a.Tp / n2 < nwarm * TL + a.flmax)
+        if (a.Tp % (TL * n2) != 0 || a.Tp / n2 < nwarm * TL)
             break;
         nseg = n2;
     }

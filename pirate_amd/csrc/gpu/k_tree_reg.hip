@@ -1,0 +1,617 @@
+// Register-resident tree dedispersion on gfx950: stage 1, and stage 2 with any subband search.
+//
+// Reference semantics: ReferenceTree (src_lib/ReferenceTree.cpp:120-345) as applied by
+// ReferenceDedisperser sophistication 1 (src_lib/ReferenceDedisperser.cpp:388-450):
+//   pass r pairs rows e = fout*2^(r+1) + dmb and o = e + 2^r (in place, bit-reversed DM):
+//     e <- c*(x_e[t - L] + x_o[t]),  o <- c*(x_e[t - L - 1] + x_o[t]),  L = bitrev(dmb, r).
+//
+// Factorization (the same identity that splits the full tree into stage 1 and stage 2):
+// a rank-DD tree over rows i = h*2^K1 + l (K1 + K2 = DD) equals
+//   phase A: 2^K2 independent rank-K1 trees over l (one per h),
+//   a delay of (2^K2 - 1 - h) * bitrev(j, K1) samples on row (h, j), j = phase-A output row,
+//   phase B: 2^K1 independent rank-K2 trees over h (one per j); final row = h'*2^K1 + j.
+// The floating-point operations are exactly those of the direct tree, so results are
+// bit-identical.
+//
+// Subbands. Stage 2 takes K2 = pf_rank, the peak finder's rank, so the rows of one phase-B tree
+// are the 2^pf_rank level-0 bands at one coarse DM pf_dm = bitrev(j, K1): every stream of that
+// DM (ReferenceTree.cpp:142-287) is a value of this tree. Band pfs of level 0 is row pfs before
+// the first pass; band pfs of level l is an output pair of pass l - 1 (pfs even), or a butterfly
+// of two neighbouring groups before that pass (pfs odd, "staggered"). A band that ends at
+// row fhi comes out (2^pf_rank - fhi) * pf_dm samples late, the phase delay of its last row:
+// that is the final lag the reference applies to the stream (ReferenceTree.cpp:42-54), so
+// streams need no further delay.
+//
+// Mapping: one workgroup per tree instance sweeps the chunk in tiles of 64 samples.
+//   Phase A: lane = time sample, one sub-tree's rows per wave in registers; a lag is a rotation
+//   across lanes, with lanes t < L taking the previous tile's values (tree_regs.hpp).
+//   Phase B: lane = two consecutive samples of a window of OV + 64 samples, OV = 2^K2, whose
+//   first OV samples only feed the lags: no histories, hence half the registers (rank 8 had
+//   spilled about 270 bytes per lane), and a shift by L and L + 1 together takes 3 lane moves
+//   for two samples instead of 4.
+// Between the phases a row goes through an LDS line that holds its last lag + OV samples and the
+// current tile; phase A appends at the end, phase B reads the OV + 64 samples at the start and
+// moves the line down by 64. Pass histories of phase A and the lines persist across chunks in an
+// HBM state buffer, double-buffered by chunk parity.
+//
+// A chunk whose length is a multiple of 32 but not of 64 ends in a half tile: its loads past
+// the chunk read zeros, its stores stop at 32 samples, and the lines move down by 32.
+//
+// Bounded by the round trips of a tile (row loads, two barriers, LDS lines), not by bytes or
+// VALU issue: rank 7 runs at 4.2-4.5 TB/s in float32, half of that in float16. No kernel spills,
+// and none calls a function: with the line offsets in a recursive constexpr function the
+// compiler called it at run time, in the tile loop, with all live registers saved around it
+// (rank 8, 4 beams of 65536 channels x 2048 samples, float16: stage 1 2.10 ms, with a table
+// 1.06 ms; the kernels that kept both phases' histories in registers 2.61 ms). Subband stage 2
+// with the passes after the first emission in LDS, a barrier after each: rank 8 4.25 -> 1.27 ms,
+// rank 6 with 34 multiplets 0.58 -> 0.18 ms.
+//
+// Segments: with few tree instances the chunk is cut into nseg runs of tiles (blockIdx.z).
+// Phase B keeps nothing from tile to tile, so a later segment only has to run phase A over the
+// tiles that fill its lines and histories (WARM tiles) before its own.
+
+#include <type_traits>
+
+#include "device_common.hpp"
+#include "kernels.hpp"
+#include "tree_regs.hpp"
+
+namespace pirate_amd {
+
+namespace {
+
+using namespace treg;
+
+constexpr int cmin(int a, int b) { return (a < b) ? a : b; }
+
+template<int DD>
+struct RegDims {
+    static constexpr int D = 1 << DD;
+    static constexpr int K1 = DD / 2, K2 = (DD + 1) / 2;
+    static constexpr int NRA = 1 << K1, NRB = 1 << K2;      // rows of a phase-A / phase-B sub-tree
+    // waves per workgroup: rank 8 one sub-tree per wave and phase in 16 waves, lower ranks 8 waves
+    static constexpr int NW = (DD >= 8) ? 16 : cmin(8, cmin(NRA, NRB));
+    static constexpr int SA = NRB / NW;                     // phase-A sub-trees per wave
+    static_assert(NRA == NW, "one phase-B sub-tree per wave");
+    static constexpr int OV = NRB;                           // window samples before the tile
+    static constexpr int WL = (OV + 64) / 2;                 // lanes of a window
+    static constexpr int T2 = NRB * (NRB - 1) / 2;
+    static constexpr int SUMB = NRA * (NRA - 1) / 2;         // sum of bitrev(j) over j
+    static constexpr int NRES = T2 * SUMB + D * OV;           // saved line samples
+    static constexpr int NSTATE = NRB * Sub<K1>::NST + NRES;
+    static constexpr int LMAX = (NRB - 1) * (NRA - 1);
+    // tiles that give a segment its lines (lag + OV samples) from outputs of phase A that no
+    // longer depend on the zero histories it started with (the first NRA - 1 samples do)
+    static constexpr int WARM = (LMAX + OV + NRA - 1 + 63) / 64;
+
+    // Line (h, j): even(lag) + OV + 64 floats, j-major, so that every line starts 8-byte aligned.
+    static constexpr int LINE0 = OV + 64;
+    static constexpr int G(int h) { return h * (NRB - 1) - h * (h - 1) / 2; }    // sum of (NRB-1-h') over h' < h
+    // start of the lines of j (a table: a function of j, even constexpr, is called at run time
+    // where j only becomes constant by unrolling)
+    struct Starts {
+        int v[NRA + 1];
+    };
+    static constexpr Starts starts()
+    {
+        Starts t{};
+        for (int j = 0; j < NRA; j++)
+            t.v[j + 1] = t.v[j] + NRB * LINE0 + brev_c(j, K1) * T2 + (brev_c(j, K1) & 1) * (NRB / 2);
+        return t;
+    }
+    static constexpr Starts CQ = starts();
+    __host__ __device__ static constexpr int lag(int h, int bj) { return (NRB - 1 - h) * bj; }
+    // start of line (h, j) within the lines of j; bj = bitrev(j, K1)
+    __host__ __device__ static constexpr int line(int h, int bj) { return h * LINE0 + bj * G(h) + (bj & 1) * ((h + 1) >> 1); }
+    static constexpr int DL_FLOATS = ((CQ.v[NRA] + 128 + 3) / 4) * 4;    // + what lanes past a window read
+    static constexpr int LDS_BYTES = 4 * DL_FLOATS;
+    // saved samples of line (h, j): lag + OV floats, j-major
+    __device__ static int res(int h, int j, int bj, int sumb) { return T2 * sumb + bj * G(h) + (j * NRB + h) * OV; }
+};
+
+// Two consecutive samples per lane.
+struct Two {
+    float x, y;
+};
+
+// v of lane - a (a = 0..NRB/2, compile-time after unrolling). Lanes below a get what feeds no
+// output (the window's first samples).
+__device__ __forceinline__ float lane_up(float v, int a, int lane)
+{
+    if (a == 0)
+        return v;
+    if (a == 1)
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));    // wave_shr:1
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(((lane - a) & 63) << 2, __float_as_int(v)));
+}
+
+// c*(e delayed by L + o) and c*(e delayed by L + 1 + o).
+__device__ __forceinline__ void butterfly(const Two &e, const Two &o, int L, int lane, Two &out0, Two &out1)
+{
+    const int a = L >> 1;
+    Two d0, d1;
+    if (L & 1) {
+        d0.x = lane_up(e.y, a + 1, lane);
+        d0.y = lane_up(e.x, a, lane);
+        d1.x = lane_up(e.x, a + 1, lane);
+        d1.y = d0.x;
+    } else {
+        d0.x = lane_up(e.x, a, lane);
+        d0.y = lane_up(e.y, a, lane);
+        d1.x = lane_up(e.y, a + 1, lane);
+        d1.y = d0.x;
+    }
+    out0.x = kRsqrt2 * (d0.x + o.x);
+    out0.y = kRsqrt2 * (d0.y + o.y);
+    out1.x = kRsqrt2 * (d1.x + o.x);
+    out1.y = kRsqrt2 * (d1.y + o.y);
+}
+
+// A wave-uniform value that the compiler must take as new: offsets formed from it are computed
+// where they are used (scalar arithmetic), not once per launch for all rows in registers that
+// the tile loop does not have.
+__device__ __forceinline__ int fresh(int x)
+{
+    asm volatile("" : "+s"(x));
+    return x;
+}
+
+// Reads the windows at the start of the lines of rows h0 .. h0 + NL - 1 of a phase-B sub-tree
+// and moves these lines down by SH samples (64, or 32 after a half tile). All by one wave, whose
+// LDS instructions execute in order; a line's loads are issued before the stores that may
+// overwrite what they read, and the loads of NL lines are in flight together.
+template<int DD, int SH, int NL, bool READ>
+__device__ __forceinline__ void take_lines(float *lj, int h0, int b, int lane, Two *v)
+{
+    using F = RegDims<DD>;
+    constexpr bool LONG = F::LMAX + F::OV > 128;
+    float2 s0[NL], s1[NL];
+#pragma unroll
+    for (int i = 0; i < NL; i++) {
+        const float2 *q = reinterpret_cast<const float2 *>(lj + F::line(h0 + i, b)) + lane;
+        if constexpr (READ) {
+            const float2 w = *q;
+            v[i].x = w.x;
+            v[i].y = w.y;
+        }
+        s0[i] = q[SH / 2];
+        if constexpr (LONG)
+            if (F::lag(h0 + i, b) + F::OV > 128)      // wave-uniform
+                s1[i] = q[SH / 2 + 64];
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < NL; i++) {
+        float2 *q = reinterpret_cast<float2 *>(lj + F::line(h0 + i, b)) + lane;
+        const int keep = F::lag(h0 + i, b) + F::OV;
+        if (2 * lane < keep)
+            q[0] = s0[i];
+        if constexpr (LONG)
+            if (128 + 2 * lane < keep)
+                q[64] = s1[i];
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ int rowlen_of(const Stage1Args &) { return 0; }
+__device__ __forceinline__ int rowlen_of(const Stage2Args &a) { return a.rowlen; }
+__device__ __forceinline__ int nband_of(const Stage1Args &, int) { return 0; }
+__device__ __forceinline__ int nband_of(const Stage2Args &a, int lev) { return a.nband[lev]; }
+
+// HC: the chunk may end in a half tile (Tp a multiple of 32, not of 64); launched only for
+// such chunks, so the common case keeps tile-uniform ring-wrap tests and no half-tile code.
+template<typename Tst, int DD, bool STAGE2, bool HC, typename Args>
+__device__ __forceinline__ void reg_tree_body(const Args &a)
+{
+    using F = RegDims<DD>;
+    using SA_ = Sub<F::K1>;
+    constexpr int D = F::D;
+    extern __shared__ __align__(16) float lbuf[];
+
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tr = blockIdx.x, b = blockIdx.y;
+    const long gbeam = long(a.beam0) + b;
+
+    const long chunk = launch_chunk(a);
+
+    // this segment's tiles
+    const int ntiles = (a.Tp + 63) >> 6;
+    const int first = int(blockIdx.z) * ntiles / a.nseg, end = (int(blockIdx.z) + 1) * ntiles / a.nseg;
+    const int start = blockIdx.z ? first - F::WARM : 0;       // >= 0: the host checks it
+
+    // state, double-buffered by chunk parity (segment 0 reads what the last segment writes)
+    const long half_state = a.state_bstride >> 1;
+    float *st = a.state + gbeam * a.state_bstride + long(tr) * F::NSTATE;
+    const float *rd = st + (chunk & 1) * half_state;
+    float *wr = st + ((chunk + 1) & 1) * half_state;
+
+    // this wave's phase-B sub-tree j: bitrev(j), its lines, and sum of bitrev(j') over j' < j
+    const int j = wid, bj = __builtin_amdgcn_readfirstlane(bitrev_dev(j, F::K1));
+    int line0 = 0, sumb = 0;
+    for (int k = 0; k < j; k++) {
+        const int bk = bitrev_dev(k, F::K1);
+        line0 += F::NRB * F::LINE0 + bk * F::T2 + (bk & 1) * (F::NRB / 2);
+        sumb += bk;
+    }
+    line0 = __builtin_amdgcn_readfirstlane(line0);
+    sumb = __builtin_amdgcn_readfirstlane(sumb);
+
+    float ha[F::SA][SA_::NH];
+    if (start == 0) {
+#pragma unroll
+        for (int s = 0; s < F::SA; s++)
+            load_hist<F::K1>(ha[s], rd + (wid + s * F::NW) * SA_::NST, lane);
+        for (int h = 0; h < F::NRB; h++) {
+            float *p = lbuf + line0 + F::line(h, bj);
+            const float *r = rd + F::NRB * SA_::NST + F::res(h, j, bj, sumb);
+            for (int q = lane; q < F::lag(h, bj) + F::OV; q += 64)
+                p[q] = r[q];
+        }
+    } else {
+#pragma unroll
+        for (int s = 0; s < F::SA; s++)
+#pragma unroll
+            for (int i = 0; i < SA_::NH; i++)
+                ha[s][i] = 0.0f;
+    }
+
+    // The wave's ring rows, one per lane: element offset, position of the next tile and capacity
+    // (32-bit, checked on the host). Stage 1 writes the rows hp*NRA + j (lane hp) of its phase-B
+    // sub-tree, stage 2 reads the rows of its phase-A sub-trees (lane s*NRA + l) at their lag.
+    // A tile that no row wraps in takes one lane read per row and scalar addresses.
+    int roff, rpos, rcap;
+    {
+        long rr, t = chunk * a.Tp + start * 64;
+        if constexpr (!STAGE2) {
+            rr = long(tr) * D + cmin(lane, F::NRB - 1) * F::NRA + j;
+        } else {
+            const int i = cmin(lane, F::SA * F::NRA - 1);
+            rr = (long((wid + (i / F::NRA) * F::NW) * F::NRA + i % F::NRA) << a.amb) + tr;
+            t -= a.row_lag[rr];
+        }
+        const long cap = a.ring.row_cap[rr];
+        roff = int(a.ring.row_off[rr]);
+        rpos = int(ring_pos(t, cap));
+        rcap = int(cap);
+    }
+    auto advance = [&](int n) {
+        rpos += n;
+        rpos -= (rpos >= rcap) ? rcap : 0;
+    };
+
+    const Tst *src;    // stage 1: this tree's input rows; stage 2: the beam's ring
+    Tst *dst;          // stage 1: the beam's ring; stage 2: the beam's peak-finder rows
+    if constexpr (!STAGE2) {
+        src = reinterpret_cast<const Tst *>(a.in) + long(b) * a.in_bstride + long(tr) * D * a.Tp;
+        dst = reinterpret_cast<Tst *>(a.ring.base) + gbeam * a.ring.bstride;
+    } else {
+        src = reinterpret_cast<const Tst *>(a.ring.base) + gbeam * a.ring.bstride;
+        dst = reinterpret_cast<Tst *>(a.sb) + gbeam * a.sb_bstride + a.tpad;
+    }
+
+    // Phase-A input rows of tile t0, issued one tile ahead and kept as loaded (raw_st) until
+    // phase A converts them; PART: a half tile, whose lanes past the chunk end take zeros
+    // (they load the last sample, so that no load sits under a per-lane branch).
+    raw_st<Tst> xa[F::SA][F::NRA];
+    auto load_a = [&](int t0, auto part) {
+        constexpr bool PART = decltype(part)::value;
+        const int tl = PART ? min(lane, a.Tp - 1 - t0) : lane;
+        const unsigned tb = unsigned(tl) * unsigned(sizeof(Tst));
+        auto at = [&](const Tst *row) {          // wave-uniform row address + 32-bit lane offset
+            return ld_raw(reinterpret_cast<const Tst *>(reinterpret_cast<const char *>(row) + tb));
+        };
+        if constexpr (!STAGE2) {
+#pragma unroll
+            for (int s = 0; s < F::SA; s++) {
+                const int h = fresh(wid + s * F::NW);
+#pragma unroll
+                for (int l = 0; l < F::NRA; l++)
+                    xa[s][l] = at(src + long(h * F::NRA + l) * a.Tp + t0);
+            }
+        } else {
+            if (!__any(rpos + 64 > rcap)) {
+                const int q = roff + rpos;
+#pragma unroll
+                for (int s = 0; s < F::SA; s++)
+#pragma unroll
+                    for (int l = 0; l < F::NRA; l++)
+                        xa[s][l] = at(src + long(__builtin_amdgcn_readlane(q, s * F::NRA + l)));
+            } else {
+#pragma unroll
+                for (int s = 0; s < F::SA; s++)
+#pragma unroll
+                    for (int l = 0; l < F::NRA; l++) {
+                        const int i = s * F::NRA + l, cap = __builtin_amdgcn_readlane(rcap, i);
+                        int q = __builtin_amdgcn_readlane(rpos, i) + tl;
+                        q -= (q >= cap) ? cap : 0;
+                        xa[s][l] = ld_raw(src + (long(__builtin_amdgcn_readlane(roff, i)) + q));
+                    }
+                asm volatile("");        // keeps the two branches' loads (and their addresses) apart
+            }
+            advance(64);
+        }
+    };
+    using Full = std::false_type;
+    using Half = std::true_type;
+
+    auto tile_step = [&](int t0, bool warm, auto half) {
+        constexpr bool HALF = decltype(half)::value;
+#pragma unroll
+        for (int s = 0; s < F::SA; s++) {
+            const int h = fresh(wid + s * F::NW);
+            float x[F::NRA];
+#pragma unroll
+            for (int l = 0; l < F::NRA; l++)
+                x[l] = (!HALF || t0 + lane < a.Tp) ? from_raw<Tst>(xa[s][l]) : 0.0f;
+            sub_passes<F::K1>(x, ha[s], lane);
+#pragma unroll
+            for (int j = 0; j < F::NRA; j++) {
+                constexpr int K1 = F::K1;
+                const int b1 = brev_c(j, K1);
+                lbuf[F::CQ.v[j] + F::line(h, b1) + F::lag(h, b1) + F::OV + lane] = x[j];
+            }
+        }
+        __syncthreads();
+        if constexpr (!HALF) {
+            if (t0 + 128 <= a.Tp)
+                load_a(t0 + 64, Full{});
+            else if (HC && t0 + 64 < a.Tp)
+                load_a(t0 + 64, Half{});
+        }
+
+        constexpr int SH = HALF ? 32 : 64;
+        float *lj = lbuf + fresh(line0);
+        const int b1 = fresh(bj);
+        constexpr int NL = cmin(4, F::NRB);
+        Two y[F::NRB];
+#pragma unroll
+        for (int h = 0; h < F::NRB; h += NL) {
+            if (warm)
+                take_lines<DD, SH, NL, false>(lj, h, b1, lane, y + h);
+            else
+                take_lines<DD, SH, NL, true>(lj, h, b1, lane, y + h);
+        }
+        if (warm) {
+            if constexpr (!STAGE2)
+                advance(64);
+            __syncthreads();
+            return;
+        }
+
+        const bool live = lane >= F::OV / 2 && lane < F::OV / 2 + SH / 2;
+        // stage 2: window lane 0's sample of multiplet 0 of this coarse DM
+        Tst *row = nullptr;
+        const int rowlen = STAGE2 ? fresh(rowlen_of(a)) : 0;
+        if constexpr (STAGE2)
+            row = dst + ((long(bitrev_dev(tr, a.amb)) << (DD - F::K2)) + b1) * a.M * rowlen + (t0 - F::OV);
+        auto emit = [&](int m, const Two &v) {
+            if constexpr (STAGE2) {
+                if (live)
+                    st2_st(row + long(m * rowlen) + unsigned(2 * lane), v.x, v.y);
+            }
+        };
+        if constexpr (STAGE2) {
+            const int nb = fresh(a.nband[0]);
+            if (nb > 0) {
+#pragma unroll
+                for (int p = 0; p < F::NRB; p++)
+                    if (p < nb)
+                        emit(p, y[p]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < F::K2; r++) {
+            const int G = 1 << r;                        // rows of a group before the pass
+            const int nb = STAGE2 ? fresh(nband_of(a, r + 1)) : 0;
+            if constexpr (STAGE2) {
+                if (nb > 1) {                 // odd bands: groups p and p + 1
+                    const int m0 = fresh(a.mband[r + 1]);
+#pragma unroll
+                    for (int p = 1; p + 1 < F::NRB / G; p += 2)
+                        if (p < nb) {
+#pragma unroll
+                            for (int x = 0; x < G; x++) {
+                                const int L = brev_c(x, r);
+                                Two o0, o1;
+                                butterfly(y[p * G + x], y[(p + 1) * G + x], L, lane, o0, o1);
+                                const int m = m0 + p * 2 * G + 2 * L;
+                                emit(m, o0);
+                                emit(m + 1, o1);
+                            }
+                        }
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < F::NRB / (2 * G); g++)
+#pragma unroll
+                for (int x = 0; x < G; x++) {
+                    const int e = g * 2 * G + x, L = brev_c(x, r);
+                    Two o0, o1;
+                    butterfly(y[e], y[e + G], L, lane, o0, o1);
+                    y[e] = o0;
+                    y[e + G] = o1;
+                }
+            if constexpr (STAGE2) {
+                if (nb > 0) {                 // even bands: the pass's outputs
+                    const int m0 = fresh(a.mband[r + 1]);
+#pragma unroll
+                    for (int g = 0; g < F::NRB / (2 * G); g++)
+                        if (2 * g < nb) {
+#pragma unroll
+                            for (int x = 0; x < G; x++) {
+                                const int e = g * 2 * G + x, L = brev_c(x, r);
+                                const int m = m0 + g * 4 * G + 2 * L;
+                                emit(m, y[e]);
+                                emit(m + 1, y[e + G]);
+                            }
+                        }
+                }
+            }
+        }
+        if constexpr (!STAGE2) {
+            // Ring positions are multiples of 64 when the chunk is, so that a tile never wraps;
+            // with half tiles they are multiples of 32 and the test is made per lane (a lane's
+            // two samples never part).
+            const int q = roff + rpos;
+#pragma unroll
+            for (int hp = 0; hp < F::NRB; hp++) {
+                if constexpr (HC) {
+                    const int cap = __builtin_amdgcn_readlane(rcap, hp);
+                    int x = __builtin_amdgcn_readlane(rpos, hp) + 2 * lane - F::OV;
+                    x -= (x >= cap) ? cap : 0;
+                    if (live)
+                        st2_st(dst + (long(__builtin_amdgcn_readlane(roff, hp)) + x), y[hp].x, y[hp].y);
+                } else {
+                    Tst *row = dst + (long(__builtin_amdgcn_readlane(q, hp)) - F::OV);
+                    if (live)
+                        st2_st(row + unsigned(2 * lane), y[hp].x, y[hp].y);
+                }
+            }
+            advance(SH);
+        }
+        __syncthreads();
+    };
+
+    if ((start + 1) * 64 <= a.Tp)
+        load_a(start * 64, Full{});
+    else if (HC)
+        load_a(start * 64, Half{});
+    const int nfull = a.Tp >> 6;
+    for (int it = start; it < min(end, nfull); it++)
+        tile_step(it * 64, it < first, Full{});
+    if constexpr (HC) {
+        if (end > nfull)
+            tile_step(nfull * 64, false, Half{});
+    }
+
+    if (blockIdx.z + 1 == gridDim.z) {
+        const int hi = (HC && (a.Tp & 63)) ? (a.Tp & 63) : 64;
+#pragma unroll
+        for (int s = 0; s < F::SA; s++)
+            save_hist<F::K1>(ha[s], wr + (wid + s * F::NW) * SA_::NST, lane, hi);
+        for (int h = 0; h < F::NRB; h++) {
+            const float *p = lbuf + line0 + F::line(h, bj);
+            float *r = wr + F::NRB * SA_::NST + F::res(h, j, bj, sumb);
+            for (int q = lane; q < F::lag(h, bj) + F::OV; q += 64)
+                r[q] = p[q];
+        }
+    }
+}
+
+template<typename Tst, int DD, bool HC>
+__global__ void __launch_bounds__(RegDims<DD>::NW * 64) __attribute__((amdgpu_waves_per_eu((DD >= 4) ? 4 : 2)))
+k_stage1(Stage1Args a)
+{
+    reg_tree_body<Tst, DD, false, HC>(a);
+}
+
+template<typename Tst, int DD, bool HC>
+__global__ void __launch_bounds__(RegDims<DD>::NW * 64) __attribute__((amdgpu_waves_per_eu((DD >= 4) ? 4 : 2)))
+k_stage2(Stage2Args a)
+{
+    reg_tree_body<Tst, DD, true, HC>(a);
+}
+
+}  // namespace
+
+
+long tree_state_nelts(int dd)
+{
+    switch (dd) {
+        case 1: return RegDims<1>::NSTATE;
+        case 2: return RegDims<2>::NSTATE;
+        case 3: return RegDims<3>::NSTATE;
+        case 4: return RegDims<4>::NSTATE;
+        case 5: return RegDims<5>::NSTATE;
+        case 6: return RegDims<6>::NSTATE;
+        case 7: return RegDims<7>::NSTATE;
+        case 8: return RegDims<8>::NSTATE;
+        default: return 0;
+    }
+}
+
+// Dynamic LDS above 64 KB (rank 8) must be allowed per kernel; gfx950 allows 160 KB.
+static void allow_lds(const void *fn, int bytes)
+{
+    if (bytes > 65536)
+        (void) hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+}
+
+// Time segments: a segment of n tiles runs n + WARM; workgroups run in rounds of as many as fit
+// on the chip (256 CUs, 16 waves and 160 KB of LDS each), and a round costs about kStart tiles
+// besides (launch, state). Takes the power of two with the shortest sum. One beam of rank 10
+// (32 instances x 32 tiles): 16 segments, stages 1 and 2 54 and 64 us -> 12 and 12 us; from some
+// 500 instances on, one segment.
+template<int DD>
+static int tree_nseg(long ninst, int Tp)
+{
+    using F = RegDims<DD>;
+    constexpr int kStart = 2;
+    constexpr long slots = 256L * cmin(16 / F::NW, 160 * 1024 / F::LDS_BYTES);
+    const int ntiles = (Tp + 63) >> 6;
+    int best = 1;
+    long cost = 0;
+    for (int n = 1; n == 1 || (ntiles / n >= cmin(F::WARM, ntiles) && n <= ntiles); n *= 2) {
+        const long rounds = (ninst * n + slots - 1) / slots;
+        const long c = rounds * ((ntiles + n - 1) / n + (n > 1 ? F::WARM : 0) + kStart);
+        if (n == 1 || c < cost) {
+            best = n;
+            cost = c;
+        }
+    }
+    return best;
+}
+
+template<int DD, typename Args>
+static void launch_tree(void (*full)(Args), void (*half)(Args), const Args &a0, hipStream_t st)
+{
+    using F = RegDims<DD>;
+    Args a = a0;
+    a.nseg = tree_nseg<DD>((1L << a.amb) * a.B, a.Tp);
+    auto *k = (a.Tp & 63) ? half : full;
+    allow_lds((const void *) k, F::LDS_BYTES);
+    hipLaunchKernelGGL(k, dim3(1 << a.amb, a.B, a.nseg), dim3(F::NW * 64), F::LDS_BYTES, st, a);
+}
+
+template<typename Tst>
+static void launch_stage1_t(const Stage1Args &a, hipStream_t st)
+{
+    switch (a.dd) {
+#define PDD_T(DDV) case DDV: launch_tree<DDV>(k_stage1<Tst, DDV, false>, k_stage1<Tst, DDV, true>, a, st); break;
+        PDD_T(1) PDD_T(2) PDD_T(3) PDD_T(4) PDD_T(5) PDD_T(6) PDD_T(7) PDD_T(8)
+#undef PDD_T
+        default: break;
+    }
+}
+
+template<typename Tst>
+static void launch_stage2_t(const Stage2Args &a, hipStream_t st)
+{
+    switch (a.dd) {
+#define PDD_T(DDV) case DDV: launch_tree<DDV>(k_stage2<Tst, DDV, false>, k_stage2<Tst, DDV, true>, a, st); break;
+        PDD_T(1) PDD_T(2) PDD_T(3) PDD_T(4) PDD_T(5) PDD_T(6) PDD_T(7) PDD_T(8)
+#undef PDD_T
+        default: break;
+    }
+}
+
+void launch_stage1(Dtype dt, const Stage1Args &a, hipStream_t st)
+{
+    switch (dt) {
+        case Dtype::float32: launch_stage1_t<float>(a, st); break;
+        case Dtype::float16: launch_stage1_t<__half>(a, st); break;
+        case Dtype::bfloat16: launch_stage1_t<__hip_bfloat16>(a, st); break;
+    }
+}
+
+void launch_stage2(Dtype dt, const Stage2Args &a, hipStream_t st)
+{
+    switch (dt) {
+        case Dtype::float32: launch_stage2_t<float>(a, st); break;
+        case Dtype::float16: launch_stage2_t<__half>(a, st); break;
+        case Dtype::bfloat16: launch_stage2_t<__hip_bfloat16>(a, st); break;
+    }
+}
+
+}  // namespace pirate_amd

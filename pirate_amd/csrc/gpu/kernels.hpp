@@ -50,55 +50,38 @@ struct Stage1Args {
     const void *in;
     long in_bstride;
     RingView ring;
-    float *state;             // per (global beam, a): tree pass history
+    float *state;             // per (global beam, a): phase-A histories and line samples
     long state_bstride;       // per beam
     int B, amb, dd, Tp, beam0;
+    int nseg = 1;             // time segments (set by launch_stage1)
     long chunk;               // chunk index (ring time = chunk*Tp + t)
     const long *chunk_dev = nullptr;   // if set, the chunk index is read here (graph replay)
 };
 
 
-// ---- stage-2 tree + subband extraction -> peak-finder input rows ----
-// Per-tree device tables built on the host (see dedisperser.cpp):
-//   main_emit[r*(D/2) + p]: first stream (pf_dm*M + m) emitted by main pair p of pass r, or -1
-//   stag[k*6 + 0..5]: (pass r, row0, row1, lag, stream s0, hist offset) staggered butterflies
-//   lvl0[k*2 + 0..1]: (row, stream) copies of the pass (dd - pf_rank) input
-//   fl[s]: final lag of stream s (applied as a write offset)
+// ---- stage-2 tree + subband streams -> peak-finder input rows ----
+// pf_rank = (dd + 1) / 2; band counts and first multiplets per subband level 0..pf_rank.
+static constexpr int kMaxPfRank = 4;
 struct Stage2Args {
     RingView ring;            // ring of the tree's primary tree
     const int *row_lag;       // (2^dd rows fc, 2^amb j) -> lag, indexed fc*2^amb + j
     void *sb;                 // (B, ndm_out, M, rowlen) peak-finder input rows
     long sb_bstride;
-    int rowlen, tpad;
-    const int *main_emit, *stag, *lvl0, *fl;
-    int nstag, nlvl0, stag_hist_nelts;
-    const int *stag_begin;    // (dd+1): staggered entries of pass r are [stag_begin[r], stag_begin[r+1])
-    int M, pf_rank;
-    float *state;             // per (global beam, j): pass history + staggered history
-    long state_bstride;
-    int B, amb, dd, Tp, beam0, amb1_dd1;   // amb1_dd1: stage-1 dd rank (ring row = fc*2^amb1_dd1 + j)
+    int rowlen, tpad, M;
+    int nband[kMaxPfRank + 1], mband[kMaxPfRank + 1];
+    float *state;             // per (global beam, j): phase-A histories and line samples
+    long state_bstride;       // per beam
+    int B, amb, dd, Tp, beam0;
+    int nseg = 1;             // time segments (set by launch_stage2)
     long chunk;
     const long *chunk_dev = nullptr;   // if set, the chunk index is read here (graph replay)
-    const int *out_stream;    // register-tree path: (2^dd) final row -> stream, or -1
-    const int *stag_goff;     // rank-8 split: staggered history offset within its row group
 };
-long stage2_state_nelts_per_tree(int dd, int stag_hist_nelts);
-int stage2_lds_bytes(int dd, int stag_hist_nelts);
-void launch_stage2(Dtype dt, const Stage2Args &a, hipStream_t st);
-// Rank-8 stage 2 with subband searches: two launches through a float32 scratch X of
-// (B, 2^amb, 256, Tp) floats; state per tree instance: split_state_nelts_per_tree(...).
-long split_state_nelts_per_tree(int stag_hist_nelts);
-int split_b_lds_bytes(int stag_hist_nelts);
-void launch_stage2_split(Dtype dt, const Stage2Args &a, float *X, hipStream_t st);
-// its part A (passes 0..3) on the register-tree code, one wave per 16-row group
-void launch_stage2_split_a_reg(Dtype dt, const Stage2Args &a, float *X, long split_nst, hipStream_t st);
 
-// ---- register-resident trees (phase A / LDS delay lines / phase B), bit-identical results ----
-// Stage 1 always; stage 2 when every stream is a final-pass output (no staggered pairs, no
-// earlier emissions). State per tree instance: fast_tree_state_nelts(dd) floats.
-long fast_tree_state_nelts(int dd);
-void launch_stage1_fast(Dtype dt, const Stage1Args &a, hipStream_t st);
-void launch_stage2_fast(Dtype dt, const Stage2Args &a, hipStream_t st);
+// State per tree instance and chunk parity: tree_state_nelts(dd) floats. state_bstride holds two
+// parities: [parity][2^amb instances].
+long tree_state_nelts(int dd);
+void launch_stage1(Dtype dt, const Stage1Args &a, hipStream_t st);
+void launch_stage2(Dtype dt, const Stage2Args &a, hipStream_t st);
 
 
 // ---- int4 dequantization: out = scale * value + offset per 256-sample (beam, freq) block ----
@@ -117,9 +100,9 @@ void launch_ringbuf_copy(void *ringbuf, const uint32_t *octuples, long noct, lon
 
 // ---- peak finder over (B, ndm_out, M, rowlen) rows -> out_max, out_argmax ----
 struct PfArgs {
-    void *sb;                 // rows [tpad history | Tp | future (max final lag)]
+    void *sb;                 // rows [tpad history | Tp]
     long sb_bstride;
-    int rowlen, tpad, flmax;
+    int rowlen, tpad;
     const int *m_to_n;        // (M)
     const float *wt;          // (B, ndm_wt, nt_wt, P, N) non-negative weights
     long wt_bstride;
