@@ -501,16 +501,40 @@ k_scorer_train(const float *P, TileSource src, const float *labels, long ntiles,
 }
 
 
+// grad[p] = the partials of parameter p added in order j = 0, 1, ... A work group takes 32
+// parameters: its threads bring up to kRedRows partials of them (128 bytes each) to LDS with all
+// loads in flight, and 32 threads add them there. Adding straight from memory, one load after the
+// other, took 121 us for 512 partials; this takes 11 us (28.5 MB).
+static constexpr int kRedCols = 32, kRedRows = 256;
+static constexpr int kRedUnroll = kRedRows * kRedCols / 256;
+
 __global__ void __launch_bounds__(256)
 k_scorer_reduce(const float *partials, int nparts, float *grad)
 {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= kNParams)
-        return;
+    __shared__ float tile[kRedRows][kRedCols];
+    const int c = threadIdx.x % kRedCols, r0 = threadIdx.x / kRedCols;
+    const int p = blockIdx.x * kRedCols + c;
+    const int pc = min(p, kNParams - 1);
     float s = 0.0f;
-    for (int j = 0; j < nparts; j++)
-        s += partials[long(j) * kNParams + p];
-    grad[p] = s;
+    for (int j0 = 0; j0 < nparts; j0 += kRedRows) {
+        float v[kRedUnroll];
+#pragma unroll
+        for (int k = 0; k < kRedUnroll; k++)
+            v[k] = partials[long(min(j0 + r0 + 8 * k, nparts - 1)) * kNParams + pc];
+        __syncthreads();                       // the previous block of rows has been added
+#pragma unroll
+        for (int k = 0; k < kRedUnroll; k++)
+            tile[r0 + 8 * k][c] = v[k];
+        __syncthreads();
+        if (threadIdx.x < kRedCols) {
+            const int n = min(kRedRows, nparts - j0);
+#pragma unroll 16
+            for (int k = 0; k < n; k++)
+                s += tile[k][c];
+        }
+    }
+    if (threadIdx.x < kRedCols && p < kNParams)
+        grad[p] = s;
 }
 
 
@@ -561,7 +585,7 @@ void launch_train(const float *params, const TileSource &src, const float *label
 
 void launch_reduce(const float *partials, int nparts, float *grad, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_scorer_reduce, dim3((kNParams + 255) / 256), dim3(256), 0, st, partials, nparts, grad);
+    hipLaunchKernelGGL(k_scorer_reduce, dim3((kNParams + kRedCols - 1) / kRedCols), dim3(256), 0, st, partials, nparts, grad);
 }
 
 void launch_adam(float *params, float *m, float *v, const float *grad, long n, float lr, float beta1, float beta2,
