@@ -23,6 +23,7 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 
 namespace pirate_amd {
 namespace scorer {
@@ -184,9 +185,9 @@ __device__ void forward_layers(const ushort_t *Xt, ushort_t *A1t, ushort_t *A2t,
     }
 }
 
-// Pooling of A_3 = relu(Y_3) over the tile: pmax, first argmax tau, pmean per channel, and the
-// logit. red: LDS scratch of 4 waves x 16 channels x 3 words; hd: 16 pmax | 16 pmean | 16 tau | logit.
-__device__ void pool_and_logit(const float y3[4][4], const float *P, float *red, float *hd)
+// Pooling of A_3 = relu(Y_3) over a wave's 64 samples: per channel the largest value, its first
+// sample and the sum, in red (4 waves x 16 channels x 3 words).
+__device__ __forceinline__ void pool_wave(const float y3[4][4], float *red)
 {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6, m = l & 15, q = l >> 4;
     for (int r = 0; r < 4; r++) {
@@ -217,6 +218,13 @@ __device__ void pool_and_logit(const float y3[4][4], const float *P, float *red,
             e[2] = sum;
         }
     }
+}
+
+// Pooling over the tile: pmax, first argmax tau, pmean per channel, and the
+// logit. red: LDS scratch of pool_wave; hd: 16 pmax | 16 pmean | 16 tau | logit.
+__device__ void pool_and_logit(const float y3[4][4], const float *P, float *red, float *hd)
+{
+    pool_wave(y3, red);
     __syncthreads();
     if (threadIdx.x < kC) {
         const int c = threadIdx.x;
@@ -251,42 +259,248 @@ __device__ __forceinline__ void load_bias(const float *P, int o, int q, float *b
 }
 
 
-__global__ void __launch_bounds__(kThreads)
+// ---- forward ----
+// One work group (4 waves) per tile, persistent over the tiles, two work groups per CU. The
+// weight fragments stay in registers (108 per lane) for the whole launch, so LDS only serves the
+// activations, which every matrix instruction reads once: that read (512 bytes per instruction,
+// 442 KB per tile) and the matrix instructions themselves (864 per tile, 16 cycles each on one
+// of the 4 SIMDs) take about 3500 cycles per tile and CU, 48 us for 8192 tiles on 256 CUs, as
+// much as reading 8192 bf16 tiles from HBM. The next tile's samples are loaded during layer 1
+// and written to LDS when layer 1 has read this tile's, and the pooled channels of a tile are
+// combined by one wave while the others start the next tile: three barriers per tile. Every
+// product is accumulated in the order of the training kernel's forward pass, so both give the
+// same bits. 8192 bf16 tiles: 131 us; with the fragments read from LDS for every product, one
+// work group per CU and scalar row loads, 555 us.
+//
+// X rows hold their 64 channels so that the 16 bytes of lane group q are channels 4q..4q+3 of two
+// neighbouring 16-channel blocks: one 16-byte read feeds two products.
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ unsigned pack_bf16(float lo, float hi)      // round to nearest even
+{
+    const f32x2 v = {lo, hi};
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+}
+
+__device__ __forceinline__ int x_slot(int cq) { return (cq >> 3) * 32 + (cq & 3) * 8 + ((cq >> 2) & 1) * 4; }
+
+// A thread's share of a tile: samples 2p, 2p + 1 (p = thread % 128) of channels 4 cq .. 4 cq + 3,
+// cq = thread / 128 + 2 g. As loaded: DT 0 float32, 1 float16, 2 bfloat16.
+template<int DT>
+struct TileLoad {
+    using E = typename std::conditional<DT == 0, unsigned, unsigned short>::type;
+    using R = typename std::conditional<DT == 0, i32x2, int>::type;
+    R r[8][4];
+
+    __device__ __forceinline__ void load(const TileSource &s, long off)
+    {
+        const int p = threadIdx.x & 127, c0 = 4 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 7);
+        const E *base = static_cast<const E *>(s.base) + off;
+        // pairs of samples in one access where the tile allows it (a tile may start anywhere)
+        const bool pairs = ((reinterpret_cast<unsigned long>(base) | (s.row_stride * sizeof(E))) & (2 * sizeof(E) - 1)) == 0;
+#pragma unroll
+        for (int g = 0; g < 8; g++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const E *q = base + long(c0 + 8 * g + j) * s.row_stride + 2 * p;
+                if (pairs) {
+                    r[g][j] = *reinterpret_cast<const R *>(q);
+                } else if constexpr (DT == 0) {
+                    r[g][j][0] = int(q[0]);
+                    r[g][j][1] = int(q[1]);
+                } else {
+                    r[g][j] = int(unsigned(q[0]) | (unsigned(q[1]) << 16));
+                }
+            }
+    }
+
+    __device__ __forceinline__ float value(int g, int j, int i) const
+    {
+        if constexpr (DT == 0)
+            return __int_as_float(r[g][j][i]);
+        else
+            return __half2float(__ushort_as_half((unsigned short) (unsigned(r[g][j]) >> (16 * i))));
+    }
+
+    __device__ __forceinline__ void store(ushort_t *Xt) const
+    {
+        const int p = threadIdx.x & 127, h = threadIdx.x >> 7;
+        const bool odd = (p >> 3) & 1;              // which sample first: spreads the rows over the banks
+#pragma unroll
+        for (int g = 0; g < 8; g++) {
+            i32x2 w[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                if constexpr (DT == 2) {
+                    const unsigned sel = i ? 0x07060302u : 0x05040100u;
+                    w[i][0] = int(__builtin_amdgcn_perm(unsigned(r[g][1]), unsigned(r[g][0]), sel));
+                    w[i][1] = int(__builtin_amdgcn_perm(unsigned(r[g][3]), unsigned(r[g][2]), sel));
+                } else {
+                    w[i][0] = int(pack_bf16(value(g, 0, i), value(g, 1, i)));
+                    w[i][1] = int(pack_bf16(value(g, 2, i), value(g, 3, i)));
+                }
+            }
+            ushort_t *row = Xt + (2 * p + kPad) * kXS + x_slot(h + 2 * g);
+            *reinterpret_cast<i32x2 *>(row + (odd ? kXS : 0)) = odd ? w[1] : w[0];
+            *reinterpret_cast<i32x2 *>(row + (odd ? 0 : kXS)) = odd ? w[0] : w[1];
+        }
+    }
+};
+
+// relu(acc + bias) rounded to bf16 -> out[(t + 4) * kAS + 4q .. 4q+3]
+__device__ __forceinline__ void store_act2(ushort_t *out, int t, int q, f32x4 acc, const float *bias)
+{
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        v[r] = fmaxf(acc[r] + bias[r], 0.0f);
+    const i32x2 w = {int(pack_bf16(v[0], v[1])), int(pack_bf16(v[2], v[3]))};
+    *reinterpret_cast<i32x2 *>(out + (t + kPad) * kAS + 4 * q) = w;
+}
+
+template<int DT>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 k_scorer_forward(const float *P, TileSource src, long ntiles, float *logits)
 {
-    __shared__ __align__(16) unsigned char smem[kXBytes + 2 * kABytes + kNFragFwd * 64 * 8 + 4 * kC * 3 * 4 + 128 * 4];
+    __shared__ __align__(16) unsigned char smem[kXBytes + 2 * kABytes];
+    __shared__ float red[4 * kC * 3];
     ushort_t *Xt = reinterpret_cast<ushort_t *>(smem);
     ushort_t *A1t = reinterpret_cast<ushort_t *>(smem + kXBytes);
     ushort_t *A2t = reinterpret_cast<ushort_t *>(smem + kXBytes + kABytes);
-    s16x4 *Wf = reinterpret_cast<s16x4 *>(smem + kXBytes + 2 * kABytes);
-    float *red = reinterpret_cast<float *>(smem + kXBytes + 2 * kABytes + kNFragFwd * 64 * 8);
-    float *hd = red + 4 * kC * 3;
+    static_assert(kXBytes >= kNFragFwd * 64 * 8, "the fragments pass through the X buffer");
 
-    const int q = (threadIdx.x & 63) >> 4;
+    const int l = threadIdx.x & 63, m = l & 15, q = l >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     float bias1[4], bias2[4], bias3[4];
     load_bias(P, ob1, q, bias1);
     load_bias(P, ob2, q, bias2);
     load_bias(P, ob3, q, bias3);
-    fill_fragments(P, Wf, kNFragFwd);
+    const float pu = P[ou + m], pv = P[ov + m], pc0 = P[oc0];
+
+    // parameters in memory order -> fragment order (through LDS) -> registers
+    s16x4 wf[kNFragFwd];
+    {
+        ushort_t *Wh = reinterpret_cast<ushort_t *>(smem);
+        for (int e = threadIdx.x; e < kC * kC0 * kK; e += kThreads) {       // W1 (co, ci, k)
+            const int k = e % kK, ci = (e / kK) % kC0, co = e / (kK * kC0);
+            Wh[((fW1 + 4 * k + (ci >> 4)) * 64 + ((ci >> 2) & 3) * 16 + co) * 4 + (ci & 3)] = f2bf(P[oW1 + e]);
+        }
+        for (int e = threadIdx.x; e < 2 * kC * kC * kK; e += kThreads) {    // W2, W3 (co, ci, k)
+            const int k = e % kK, ci = (e / kK) % kC, co = (e / (kK * kC)) % kC, layer = e / (kK * kC * kC);
+            Wh[((fW2 + layer * kK + k) * 64 + (ci >> 2) * 16 + co) * 4 + (ci & 3)] = f2bf(P[oW2 + e]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int f = 0; f < kNFragFwd; f++)
+            wf[f] = ld4(Wh + (f * 64 + l) * 4);
+        __syncthreads();
+    }
     zero_halo(Xt, kXS);
     zero_halo(A1t, kAS);
     zero_halo(A2t, kAS);
 
-    for (long n = blockIdx.x; n < ntiles; n += gridDim.x) {
-        long off = 0;
-        if (!tile_origin(src, n, off)) {            // uniform over the work group
+    // the next tile of this work group in the valid range (the others get NaN): uniform
+    auto next = [&](long n, long &off) {
+        while (n < ntiles && !tile_origin(src, n, off)) {
             if (threadIdx.x == 0)
                 logits[n] = __int_as_float(0x7fc00000);
-            continue;
+            n += gridDim.x;
         }
-        __syncthreads();                            // previous tile's readers of Xt / A1t / A2t are done
-        load_tile(src, off, Xt);
+        return n;
+    };
+
+    TileLoad<DT> x;
+    long off = 0;
+    long n = next(blockIdx.x, off);
+    if (n < ntiles) {
+        x.load(src, off);
+        x.store(Xt);
+    }
+    __syncthreads();
+    while (n < ntiles) {
+        const long n2 = next(n + gridDim.x, off);
+        if (n2 < ntiles)
+            x.load(src, off);
+
+        f32x4 acc[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            acc[i] = {0.0f, 0.0f, 0.0f, 0.0f};
+        const ushort_t *xr = Xt + (64 * w + m) * kXS + 8 * q;
+#pragma unroll
+        for (int k = 0; k < kK; k++)
+#pragma unroll
+            for (int cp = 0; cp < 2; cp++) {
+                i32x4 v[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    v[i] = *reinterpret_cast<const i32x4 *>(xr + (16 * i + k) * kXS + 32 * cp);
+#pragma unroll
+                for (int c = 0; c < 2; c++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const i32x2 h = {v[i][2 * c], v[i][2 * c + 1]};
+                        acc[i] = mfma16(wf[fW1 + 4 * k + 2 * cp + c], __builtin_bit_cast(s16x4, h), acc[i]);
+                    }
+            }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            store_act2(A1t, 64 * w + 16 * i + m, q, acc[i], bias1);
         __syncthreads();
+
+        if (n2 < ntiles)
+            x.store(Xt);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            acc[i] = {0.0f, 0.0f, 0.0f, 0.0f};
+        const ushort_t *ar = A1t + (64 * w + m) * kAS + 4 * q;
+#pragma unroll
+        for (int k = 0; k < kK; k++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                acc[i] = mfma16(wf[fW2 + k], ld4(ar + (16 * i + k) * kAS), acc[i]);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            store_act2(A2t, 64 * w + 16 * i + m, q, acc[i], bias2);
+        __syncthreads();
+
         float y3[4][4];
-        forward_layers(Xt, A1t, A2t, Wf, bias1, bias2, bias3, y3);
-        pool_and_logit(y3, P, red, hd);
-        if (threadIdx.x == 0)
-            logits[n] = hd[3 * kC];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            acc[i] = {0.0f, 0.0f, 0.0f, 0.0f};
+        ar = A2t + (64 * w + m) * kAS + 4 * q;
+#pragma unroll
+        for (int k = 0; k < kK; k++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                acc[i] = mfma16(wf[fW3 + k], ld4(ar + (16 * i + k) * kAS), acc[i]);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                y3[i][r] = acc[i][r] + bias3[r];
+        pool_wave(y3, red);
+        __syncthreads();
+        if (w == 0) {
+            // lane m: channel m over the waves; then the head, channels in order
+            float best = red[m * 3], sum = red[m * 3 + 2];
+#pragma unroll
+            for (int ww = 1; ww < 4; ww++) {
+                best = (red[(ww * kC + m) * 3] > best) ? red[(ww * kC + m) * 3] : best;
+                sum += red[(ww * kC + m) * 3 + 2];
+            }
+            const float t = pu * best + pv * (sum * (1.0f / kT));
+            float z = pc0;
+#pragma unroll
+            for (int c = 0; c < kC; c++)
+                z += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t), c));
+            if (l == 0)
+                logits[n] = z;
+        }
+        n = n2;
     }
 }
 
@@ -563,16 +777,20 @@ int train_nparts(long ntiles, int max_parts)
 
 static int forward_blocks(long ntiles)
 {
-    // one resident work group per CU (LDS-limited); 4 rounds of 256 CUs, then grid-stride
-    return int(ntiles < 1024 ? ntiles : 1024);
+    // two resident work groups per CU (registers), persistent over the tiles
+    return int(ntiles < 512 ? ntiles : 512);
 }
 
 void launch_forward(const float *params, const TileSource &src, long ntiles, float *logits, hipStream_t st)
 {
     if (ntiles <= 0)
         return;
-    hipLaunchKernelGGL(k_scorer_forward, dim3(forward_blocks(ntiles)), dim3(kThreads), 0, st, params, src, ntiles,
-                       logits);
+    const dim3 grid(forward_blocks(ntiles)), block(kThreads);
+    switch (src.dtype) {
+        case kFloat32: hipLaunchKernelGGL(k_scorer_forward<0>, grid, block, 0, st, params, src, ntiles, logits); break;
+        case kFloat16: hipLaunchKernelGGL(k_scorer_forward<1>, grid, block, 0, st, params, src, ntiles, logits); break;
+        default: hipLaunchKernelGGL(k_scorer_forward<2>, grid, block, 0, st, params, src, ntiles, logits); break;
+    }
 }
 
 void launch_train(const float *params, const TileSource &src, const float *labels, long ntiles, float inv_n,
