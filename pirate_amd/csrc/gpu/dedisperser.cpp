@@ -295,7 +295,7 @@ void GpuDedisperser::allocate()
                 long r = a1 * pow2(dd1) + j;
                 if (minlag >= 0 && max_gpu_clag < (1L << 40))
                     kr[r] = std::max(0L, minlag / Tp - max_gpu_clag);
-                cap[r] = align_up(maxlag - kr[r] * Tp + Tp, 64);
+                cap[r] = align_up(maxlag - kr[r] * Tp + Tp + kTreeOverlap, 64);
                 off[r] = tot;
                 tot += cap[r];
             }

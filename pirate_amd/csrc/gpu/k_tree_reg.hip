@@ -22,33 +22,40 @@
 // that is the final lag the reference applies to the stream (ReferenceTree.cpp:42-54), so
 // streams need no further delay.
 //
-// Mapping: one workgroup per tree instance sweeps the chunk in tiles of 64 samples.
-//   Phase A: lane = time sample, one sub-tree's rows per wave in registers; a lag is a rotation
-//   across lanes, with lanes t < L taking the previous tile's values (tree_regs.hpp).
-//   Phase B: lane = two consecutive samples of a window of OV + 64 samples, OV = 2^K2, whose
-//   first OV samples only feed the lags: no histories, hence half the registers (rank 8 had
-//   spilled about 270 bytes per lane), and a shift by L and L + 1 together takes 3 lane moves
-//   for two samples instead of 4.
+// Mapping: one workgroup per tree instance sweeps the chunk in tiles of U = 96 samples (rank 8:
+// 64), one sub-tree's rows per wave in registers. Both phases work in windows: lane = two
+// consecutive samples, and the first OVA = 2^K1 (phase A) or OV = 2^K2 (phase B) samples of a
+// window come before the tile and only feed the lags. So there are no histories to hold or to
+// select from, and a shift by L and L + 1 together takes 3 lane moves for two samples instead of
+// 4. 96 samples fill 52 to 56 of 64 lanes, tiles of 64 no more than 40.
+//   Rank 8 has LDS for tiles of 64 to 80 samples only; there phase A holds lane = one sample,
+// with lanes t < L taking the previous tile's values (tree_regs.hpp).
 // Between the phases a row goes through an LDS line that holds its last lag + OV samples and the
-// current tile; phase A appends at the end, phase B reads the OV + 64 samples at the start and
-// moves the line down by 64. Pass histories of phase A and the lines persist across chunks in an
-// HBM state buffer, double-buffered by chunk parity.
+// current tile; phase A appends at the end, phase B reads the OV + U samples at the start and
+// moves the line down by U. The lines persist across chunks in an HBM state buffer,
+// double-buffered by chunk parity, with the last OVA input samples of stage 1 (stage 2 finds
+// its own in the ring, whose rows are OVA samples longer) or rank 8's histories.
 //
-// A chunk whose length is a multiple of 32 but not of 64 ends in a half tile: its loads past
-// the chunk read zeros, its stores stop at 32 samples, and the lines move down by 32.
+// A chunk that is no multiple of U ends in a smaller tile (a multiple of 32 samples): its loads
+// stay inside the chunk, its stores stop at the chunk's end, and the lines move down by its
+// length.
 //
-// Bounded by the round trips of a tile (row loads, two barriers, LDS lines), not by bytes or
-// VALU issue: rank 7 runs at 4.2-4.5 TB/s in float32, half of that in float16. No kernel spills,
-// and none calls a function: with the line offsets in a recursive constexpr function the
-// compiler called it at run time, in the tile loop, with all live registers saved around it
-// (rank 8, 4 beams of 65536 channels x 2048 samples, float16: stage 1 2.10 ms, with a table
-// 1.06 ms; the kernels that kept both phases' histories in registers 2.61 ms). Subband stage 2
-// with the passes after the first emission in LDS, a barrier after each: rank 8 4.25 -> 1.27 ms,
-// rank 6 with 34 multiplets 0.58 -> 0.18 ms.
+// Bounded by VALU issue (about 65% busy in float16) and the round trips of a tile (row loads,
+// two barriers, LDS lines), not by bytes: rank 7 runs at 4.2-4.6 TB/s in float32, 2.8-3.0 in
+// float16. 16 beams of 16384 channels x 2048 samples, stages 1 and 2 (rank 7): float16 0.83 and
+// 0.86 ms with tiles of 64 and phase-A histories, 0.72 and 0.77 ms now; float32 0.99 and 0.95,
+// 1.01 and 0.94 ms. Rank 8 (4 beams of 65536 channels, float16) with histories 1.05 and 1.08 ms,
+// in windows and tiles of 64 1.16 and 1.26, of 80 1.07 and 1.14; its subband stage 2 1.26, 1.48
+// and 1.61 ms (rows of 80 16-bit samples start inside 64-byte blocks).
+// No kernel spills, and none calls a function: with the line offsets in a recursive constexpr
+// function the compiler called it at run time, in the tile loop, with all live registers saved
+// around it (rank 8 stage 1 2.10 ms, with a table 1.06 ms; the kernels that kept both phases'
+// histories in registers 2.61 ms). Subband stage 2 with the passes after the first emission in
+// LDS, a barrier after each: rank 8 4.25 ms, rank 6 with 34 multiplets 0.58 -> 0.18 ms.
 //
 // Segments: with few tree instances the chunk is cut into nseg runs of tiles (blockIdx.z).
 // Phase B keeps nothing from tile to tile, so a later segment only has to run phase A over the
-// tiles that fill its lines and histories (WARM tiles) before its own.
+// tiles that fill its lines (and histories) before its own (WARM tiles).
 
 #include <type_traits>
 
@@ -73,19 +80,30 @@ struct RegDims {
     static constexpr int NW = (DD >= 8) ? 16 : cmin(8, cmin(NRA, NRB));
     static constexpr int SA = NRB / NW;                     // phase-A sub-trees per wave
     static_assert(NRA == NW, "one phase-B sub-tree per wave");
-    static constexpr int OV = NRB;                           // window samples before the tile
-    static constexpr int WL = (OV + 64) / 2;                 // lanes of a window
+    // Phase A in windows, as phase B, or (rank 8) one sample per lane with histories: where LDS
+    // keeps the tile at 64 samples, 16 more in each window cost more than the histories (figures
+    // at the top).
+    static constexpr bool HIST = DD >= 8;
+    static constexpr int S = HIST ? 1 : 2;                  // phase-A samples per lane
+    // samples per tile: for 2 samples per lane as many as 64 lanes and two workgroups' lines in
+    // LDS take. A multiple of 32, as are chunks, so that a chunk's last tile is one as well.
+    static constexpr int U = HIST ? 64 : 96;
+    static constexpr int OVA = (K1 > 0 && !HIST) ? NRA : 0, OV = NRB;    // window samples before the tile
+    static constexpr int WLA = (OVA + U) / S, WL = (OV + U) / 2;         // lanes of a window
     static constexpr int T2 = NRB * (NRB - 1) / 2;
     static constexpr int SUMB = NRA * (NRA - 1) / 2;         // sum of bitrev(j) over j
     static constexpr int NRES = T2 * SUMB + D * OV;           // saved line samples
-    static constexpr int NSTATE = NRB * Sub<K1>::NST + NRES;
+    // and the histories, or the last input samples (stage 1)
+    static constexpr int NSTATE = NRES + (HIST ? NRB * Sub<K1>::NST : D * OVA);
     static constexpr int LMAX = (NRB - 1) * (NRA - 1);
-    // tiles that give a segment its lines (lag + OV samples) from outputs of phase A that no
-    // longer depend on the zero histories it started with (the first NRA - 1 samples do)
-    static constexpr int WARM = (LMAX + OV + NRA - 1 + 63) / 64;
+    // tiles that fill a segment's lines (lag + OV samples), with histories from outputs that no
+    // longer depend on the zeros it started with (the first NRA - 1 samples do)
+    static constexpr int WARM = (LMAX + OV + (HIST ? NRA - 1 : 0) + U - 1) / U;
+    static_assert(WLA <= 64 && WL <= 64, "a window fits a wave");
+    static_assert(OVA <= kTreeOverlap, "ring capacities");
 
-    // Line (h, j): even(lag) + OV + 64 floats, j-major, so that every line starts 8-byte aligned.
-    static constexpr int LINE0 = OV + 64;
+    // Line (h, j): even(lag) + OV + U floats, j-major, so that every line starts 8-byte aligned.
+    static constexpr int LINE0 = OV + U;
     static constexpr int G(int h) { return h * (NRB - 1) - h * (h - 1) / 2; }    // sum of (NRB-1-h') over h' < h
     // start of the lines of j (a table: a function of j, even constexpr, is called at run time
     // where j only becomes constant by unrolling)
@@ -103,8 +121,10 @@ struct RegDims {
     __host__ __device__ static constexpr int lag(int h, int bj) { return (NRB - 1 - h) * bj; }
     // start of line (h, j) within the lines of j; bj = bitrev(j, K1)
     __host__ __device__ static constexpr int line(int h, int bj) { return h * LINE0 + bj * G(h) + (bj & 1) * ((h + 1) >> 1); }
-    static constexpr int DL_FLOATS = ((CQ.v[NRA] + 128 + 3) / 4) * 4;    // + what lanes past a window read
+    // + what lanes past a window read
+    static constexpr int DL_FLOATS = ((CQ.v[NRA] + ((LMAX + OV > 128) ? 192 : 128) + 3) / 4) * 4;
     static constexpr int LDS_BYTES = 4 * DL_FLOATS;
+    static_assert(LDS_BYTES <= 160 * 1024, "LDS of a CU");
     // saved samples of line (h, j): lag + OV floats, j-major
     __device__ static int res(int h, int j, int bj, int sumb) { return T2 * sumb + bj * G(h) + (j * NRB + h) * OV; }
 };
@@ -157,11 +177,11 @@ __device__ __forceinline__ int fresh(int x)
 }
 
 // Reads the windows at the start of the lines of rows h0 .. h0 + NL - 1 of a phase-B sub-tree
-// and moves these lines down by SH samples (64, or 32 after a half tile). All by one wave, whose
-// LDS instructions execute in order; a line's loads are issued before the stores that may
-// overwrite what they read, and the loads of NL lines are in flight together.
-template<int DD, int SH, int NL, bool READ>
-__device__ __forceinline__ void take_lines(float *lj, int h0, int b, int lane, Two *v)
+// and moves these lines down by sh samples (U, or the chunk's last samples: even). All by one
+// wave, whose LDS instructions execute in order; a line's loads are issued before the stores that
+// may overwrite what they read, and the loads of NL lines are in flight together.
+template<int DD, int NL, bool READ>
+__device__ __forceinline__ void take_lines(float *lj, int h0, int b, int lane, int sh, Two *v)
 {
     using F = RegDims<DD>;
     constexpr bool LONG = F::LMAX + F::OV > 128;
@@ -174,10 +194,10 @@ __device__ __forceinline__ void take_lines(float *lj, int h0, int b, int lane, T
             v[i].x = w.x;
             v[i].y = w.y;
         }
-        s0[i] = q[SH / 2];
+        s0[i] = q[sh / 2];
         if constexpr (LONG)
             if (F::lag(h0 + i, b) + F::OV > 128)      // wave-uniform
-                s1[i] = q[SH / 2 + 64];
+                s1[i] = q[sh / 2 + 64];
     }
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -193,19 +213,43 @@ __device__ __forceinline__ void take_lines(float *lj, int h0, int b, int lane, T
     __builtin_amdgcn_wave_barrier();
 }
 
+// S (1 or 2) consecutive samples as loaded, at any element alignment.
+template<typename Tst, int S>
+struct RawS {
+    raw_st<Tst> v;
+    __device__ __forceinline__ void load(const Tst *p) { v = ld_raw(p); }
+    __device__ __forceinline__ void set(const Tst *p, const Tst *) { v = ld_raw(p); }
+};
+template<>
+struct RawS<float, 2> {
+    typedef float V __attribute__((ext_vector_type(2), aligned(4)));
+    V v;
+    __device__ __forceinline__ void load(const float *p) { v = *reinterpret_cast<const V *>(p); }
+    __device__ __forceinline__ void set(const float *p, const float *q) { v = V{*p, *q}; }
+    __device__ __forceinline__ Two get() const { return Two{v.x, v.y}; }
+};
+template<typename T16>
+struct RawTwo16 {
+    typedef unsigned V __attribute__((aligned(2)));
+    unsigned v;
+    __device__ __forceinline__ void load(const T16 *p) { v = *reinterpret_cast<const V *>(p); }
+    __device__ __forceinline__ void set(const T16 *p, const T16 *q) { v = ld_raw(p) | (ld_raw(q) << 16); }
+    __device__ __forceinline__ Two get() const { return Two{from_raw<T16>(v & 0xffffu), from_raw<T16>(v >> 16)}; }
+};
+template<> struct RawS<__half, 2> : RawTwo16<__half> { };
+template<> struct RawS<__hip_bfloat16, 2> : RawTwo16<__hip_bfloat16> { };
+
 __device__ __forceinline__ int rowlen_of(const Stage1Args &) { return 0; }
 __device__ __forceinline__ int rowlen_of(const Stage2Args &a) { return a.rowlen; }
 __device__ __forceinline__ int nband_of(const Stage1Args &, int) { return 0; }
 __device__ __forceinline__ int nband_of(const Stage2Args &a, int lev) { return a.nband[lev]; }
 
-// HC: the chunk may end in a half tile (Tp a multiple of 32, not of 64); launched only for
-// such chunks, so the common case keeps tile-uniform ring-wrap tests and no half-tile code.
-template<typename Tst, int DD, bool STAGE2, bool HC, typename Args>
+template<typename Tst, int DD, bool STAGE2, typename Args>
 __device__ __forceinline__ void reg_tree_body(const Args &a)
 {
     using F = RegDims<DD>;
     using SA_ = Sub<F::K1>;
-    constexpr int D = F::D;
+    constexpr int D = F::D, U = F::U;
     extern __shared__ __align__(16) float lbuf[];
 
     const int lane = threadIdx.x & 63;
@@ -216,7 +260,7 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
     const long chunk = launch_chunk(a);
 
     // this segment's tiles
-    const int ntiles = (a.Tp + 63) >> 6;
+    const int ntiles = (a.Tp + U - 1) / U;
     const int first = int(blockIdx.z) * ntiles / a.nseg, end = (int(blockIdx.z) + 1) * ntiles / a.nseg;
     const int start = blockIdx.z ? first - F::WARM : 0;       // >= 0: the host checks it
 
@@ -236,39 +280,43 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
     }
     line0 = __builtin_amdgcn_readfirstlane(line0);
     sumb = __builtin_amdgcn_readfirstlane(sumb);
-
-    float ha[F::SA][SA_::NH];
     if (start == 0) {
-#pragma unroll
-        for (int s = 0; s < F::SA; s++)
-            load_hist<F::K1>(ha[s], rd + (wid + s * F::NW) * SA_::NST, lane);
         for (int h = 0; h < F::NRB; h++) {
             float *p = lbuf + line0 + F::line(h, bj);
-            const float *r = rd + F::NRB * SA_::NST + F::res(h, j, bj, sumb);
+            const float *r = rd + F::res(h, j, bj, sumb);
             for (int q = lane; q < F::lag(h, bj) + F::OV; q += 64)
                 p[q] = r[q];
         }
-    } else {
-#pragma unroll
-        for (int s = 0; s < F::SA; s++)
-#pragma unroll
-            for (int i = 0; i < SA_::NH; i++)
-                ha[s][i] = 0.0f;
     }
 
-    // The wave's ring rows, one per lane: element offset, position of the next tile and capacity
-    // (32-bit, checked on the host). Stage 1 writes the rows hp*NRA + j (lane hp) of its phase-B
-    // sub-tree, stage 2 reads the rows of its phase-A sub-trees (lane s*NRA + l) at their lag.
-    // A tile that no row wraps in takes one lane read per row and scalar addresses.
+    float ha[F::HIST ? F::SA : 1][F::HIST ? SA_::NH : 1];
+    if constexpr (F::HIST) {
+#pragma unroll
+        for (int s = 0; s < F::SA; s++) {
+            if (start == 0) {
+                load_hist<F::K1>(ha[s], rd + F::NRES + (wid + s * F::NW) * SA_::NST, lane);
+            } else {
+#pragma unroll
+                for (int i = 0; i < SA_::NH; i++)
+                    ha[s][i] = 0.0f;
+            }
+        }
+    }
+
+    // The wave's ring rows, one per lane: element offset, position and capacity (32-bit, checked
+    // on the host). Stage 1 writes the rows hp*NRA + j (lane hp) of its phase-B sub-tree, at the
+    // position of the next tile; stage 2 reads the rows of its phase-A sub-trees (lane s*NRA + l) at
+    // their lag, from the start of the next tile's window. A tile that no row wraps in takes one
+    // lane read per row and scalar addresses.
     int roff, rpos, rcap;
     {
-        long rr, t = chunk * a.Tp + start * 64;
+        long rr, t = chunk * a.Tp + start * U;
         if constexpr (!STAGE2) {
             rr = long(tr) * D + cmin(lane, F::NRB - 1) * F::NRA + j;
         } else {
             const int i = cmin(lane, F::SA * F::NRA - 1);
             rr = (long((wid + (i / F::NRA) * F::NW) * F::NRA + i % F::NRA) << a.amb) + tr;
-            t -= a.row_lag[rr];
+            t -= a.row_lag[rr] + F::OVA;
         }
         const long cap = a.ring.row_cap[rr];
         roff = int(a.ring.row_off[rr]);
@@ -290,77 +338,120 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
         dst = reinterpret_cast<Tst *>(a.sb) + gbeam * a.sb_bstride + a.tpad;
     }
 
-    // Phase-A input rows of tile t0, issued one tile ahead and kept as loaded (raw_st) until
-    // phase A converts them; PART: a half tile, whose lanes past the chunk end take zeros
-    // (they load the last sample, so that no load sits under a per-lane branch).
-    raw_st<Tst> xa[F::SA][F::NRA];
-    auto load_a = [&](int t0, auto part) {
-        constexpr bool PART = decltype(part)::value;
-        const int tl = PART ? min(lane, a.Tp - 1 - t0) : lane;
-        const unsigned tb = unsigned(tl) * unsigned(sizeof(Tst));
-        auto at = [&](const Tst *row) {          // wave-uniform row address + 32-bit lane offset
-            return ld_raw(reinterpret_cast<const Tst *>(reinterpret_cast<const char *>(row) + tb));
-        };
+    // Phase-A windows of tile t0, issued one tile ahead and kept as loaded until phase A converts
+    // them. Lanes past the window (or the chunk) load its last samples. Stage 1 clamps what lies
+    // before the chunk to its start: phase A takes the saved samples there.
+    RawS<Tst, F::S> xa[F::SA][F::NRA];
+    auto load_a = [&](int t0) {
+        const int wlen = F::OVA + min(U, a.Tp - t0);           // a capacity holds a whole window
+        const int i = min(F::S * lane, wlen - F::S);
         if constexpr (!STAGE2) {
+            const unsigned tb = unsigned(max(t0 - F::OVA + i, 0)) * unsigned(sizeof(Tst));
 #pragma unroll
             for (int s = 0; s < F::SA; s++) {
                 const int h = fresh(wid + s * F::NW);
 #pragma unroll
-                for (int l = 0; l < F::NRA; l++)
-                    xa[s][l] = at(src + long(h * F::NRA + l) * a.Tp + t0);
+                for (int l = 0; l < F::NRA; l++) {
+                    const Tst *row = src + long(h * F::NRA + l) * a.Tp;
+                    xa[s][l].load(reinterpret_cast<const Tst *>(reinterpret_cast<const char *>(row) + tb));
+                }
             }
         } else {
-            if (!__any(rpos + 64 > rcap)) {
+            const unsigned tb = unsigned(i) * unsigned(sizeof(Tst));
+            if (!__any(rpos + wlen > rcap)) {
                 const int q = roff + rpos;
 #pragma unroll
                 for (int s = 0; s < F::SA; s++)
 #pragma unroll
-                    for (int l = 0; l < F::NRA; l++)
-                        xa[s][l] = at(src + long(__builtin_amdgcn_readlane(q, s * F::NRA + l)));
+                    for (int l = 0; l < F::NRA; l++) {
+                        const Tst *row = src + long(__builtin_amdgcn_readlane(q, s * F::NRA + l));
+                        xa[s][l].load(reinterpret_cast<const Tst *>(reinterpret_cast<const char *>(row) + tb));
+                    }
             } else {
 #pragma unroll
                 for (int s = 0; s < F::SA; s++)
 #pragma unroll
                     for (int l = 0; l < F::NRA; l++) {
-                        const int i = s * F::NRA + l, cap = __builtin_amdgcn_readlane(rcap, i);
-                        int q = __builtin_amdgcn_readlane(rpos, i) + tl;
-                        q -= (q >= cap) ? cap : 0;
-                        xa[s][l] = ld_raw(src + (long(__builtin_amdgcn_readlane(roff, i)) + q));
+                        const int k = s * F::NRA + l, cap = __builtin_amdgcn_readlane(rcap, k);
+                        const Tst *row = src + long(__builtin_amdgcn_readlane(roff, k));
+                        const int q0 = __builtin_amdgcn_readlane(rpos, k) + i, q1 = q0 + 1;
+                        xa[s][l].set(row + (q0 - ((q0 >= cap) ? cap : 0)), row + (q1 - ((q1 >= cap) ? cap : 0)));
                     }
                 asm volatile("");        // keeps the two branches' loads (and their addresses) apart
             }
-            advance(64);
+            advance(U);
         }
     };
-    using Full = std::false_type;
-    using Half = std::true_type;
 
-    auto tile_step = [&](int t0, bool warm, auto half) {
-        constexpr bool HALF = decltype(half)::value;
+    // Tile t0 of nv samples: U, or what is left of the chunk (a multiple of 32).
+    using Full = std::integral_constant<int, U>;
+    auto tile_step = [&](int t0, bool warm, auto nv_) {
+        const int nv = nv_;
 #pragma unroll
         for (int s = 0; s < F::SA; s++) {
             const int h = fresh(wid + s * F::NW);
-            float x[F::NRA];
+            if constexpr (F::HIST) {
+                float x[F::NRA];
 #pragma unroll
-            for (int l = 0; l < F::NRA; l++)
-                x[l] = (!HALF || t0 + lane < a.Tp) ? from_raw<Tst>(xa[s][l]) : 0.0f;
-            sub_passes<F::K1>(x, ha[s], lane);
+                for (int l = 0; l < F::NRA; l++)
+                    x[l] = from_raw<Tst>(xa[s][l].v);
+                sub_passes<F::K1>(x, ha[s], lane);
 #pragma unroll
-            for (int j = 0; j < F::NRA; j++) {
-                constexpr int K1 = F::K1;
-                const int b1 = brev_c(j, K1);
-                lbuf[F::CQ.v[j] + F::line(h, b1) + F::lag(h, b1) + F::OV + lane] = x[j];
+                for (int jj = 0; jj < F::NRA; jj++) {
+                    constexpr int K1 = F::K1;
+                    const int b1 = brev_c(jj, K1);
+                    lbuf[F::CQ.v[jj] + F::line(h, b1) + F::lag(h, b1) + F::OV + lane] = x[jj];
+                }
+            } else {
+                Two x[F::NRA];
+#pragma unroll
+                for (int l = 0; l < F::NRA; l++)
+                    x[l] = xa[s][l].get();
+                if constexpr (!STAGE2 && F::OVA > 0) {
+                    // the input samples before the chunk, and the chunk's last ones for the next
+                    if (t0 == 0 && lane < F::OVA / 2) {
+#pragma unroll
+                        for (int l = 0; l < F::NRA; l++) {
+                            const float2 y = *reinterpret_cast<const float2 *>(rd + F::NRES + (h * F::NRA + l) * F::OVA + 2 * lane);
+                            x[l] = Two{y.x, y.y};
+                        }
+                    }
+                    const int k = 2 * lane - nv;
+                    if (t0 + nv == a.Tp && k >= 0 && k < F::OVA) {
+#pragma unroll
+                        for (int l = 0; l < F::NRA; l++)
+                            *reinterpret_cast<float2 *>(wr + F::NRES + (h * F::NRA + l) * F::OVA + k) = make_float2(x[l].x, x[l].y);
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < F::K1; r++) {
+                    const int G = 1 << r;
+#pragma unroll
+                    for (int e0 = 0; e0 < F::NRA; e0 += 2 * G)
+#pragma unroll
+                        for (int d = 0; d < G; d++) {
+                            Two o0, o1;
+                            butterfly(x[e0 + d], x[e0 + d + G], brev_c(d, r), lane, o0, o1);
+                            x[e0 + d] = o0;
+                            x[e0 + d + G] = o1;
+                        }
+                }
+                if (lane >= F::OVA / 2 && lane < F::WLA) {
+#pragma unroll
+                    for (int jj = 0; jj < F::NRA; jj++) {
+                        constexpr int K1 = F::K1;
+                        const int b1 = brev_c(jj, K1);
+                        float *p = lbuf + (F::CQ.v[jj] + F::line(h, b1) + F::lag(h, b1) + F::OV - F::OVA) + 2 * lane;
+                        p[0] = x[jj].x;
+                        p[1] = x[jj].y;
+                    }
+                }
             }
         }
         __syncthreads();
-        if constexpr (!HALF) {
-            if (t0 + 128 <= a.Tp)
-                load_a(t0 + 64, Full{});
-            else if (HC && t0 + 64 < a.Tp)
-                load_a(t0 + 64, Half{});
-        }
+        if (t0 + U < a.Tp)
+            load_a(t0 + U);
 
-        constexpr int SH = HALF ? 32 : 64;
         float *lj = lbuf + fresh(line0);
         const int b1 = fresh(bj);
         constexpr int NL = cmin(4, F::NRB);
@@ -368,32 +459,30 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
 #pragma unroll
         for (int h = 0; h < F::NRB; h += NL) {
             if (warm)
-                take_lines<DD, SH, NL, false>(lj, h, b1, lane, y + h);
+                take_lines<DD, NL, false>(lj, h, b1, lane, nv, y + h);
             else
-                take_lines<DD, SH, NL, true>(lj, h, b1, lane, y + h);
+                take_lines<DD, NL, true>(lj, h, b1, lane, nv, y + h);
         }
         if (warm) {
             if constexpr (!STAGE2)
-                advance(64);
+                advance(U);
             __syncthreads();
             return;
         }
 
-        const bool live = lane >= F::OV / 2 && lane < F::OV / 2 + SH / 2;
+        const bool live = lane >= F::OV / 2 && lane < (F::OV + nv) / 2;
         // stage 2: window lane 0's sample of multiplet 0 of this coarse DM
         Tst *row = nullptr;
         const int rowlen = STAGE2 ? fresh(rowlen_of(a)) : 0;
         if constexpr (STAGE2)
             row = dst + ((long(bitrev_dev(tr, a.amb)) << (DD - F::K2)) + b1) * a.M * rowlen + (t0 - F::OV);
         auto emit = [&](int m, const Two &v) {
-            if constexpr (STAGE2) {
-                if (live)
-                    st2_st(row + long(m * rowlen) + unsigned(2 * lane), v.x, v.y);
-            }
+            if constexpr (STAGE2)
+                st2_st(row + long(m * rowlen) + unsigned(2 * lane), v.x, v.y);
         };
         if constexpr (STAGE2) {
             const int nb = fresh(a.nband[0]);
-            if (nb > 0) {
+            if (nb > 0 && live) {
 #pragma unroll
                 for (int p = 0; p < F::NRB; p++)
                     if (p < nb)
@@ -405,7 +494,7 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
             const int G = 1 << r;                        // rows of a group before the pass
             const int nb = STAGE2 ? fresh(nband_of(a, r + 1)) : 0;
             if constexpr (STAGE2) {
-                if (nb > 1) {                 // odd bands: groups p and p + 1
+                if (nb > 1) {                            // odd bands: groups p and p + 1
                     const int m0 = fresh(a.mband[r + 1]);
 #pragma unroll
                     for (int p = 1; p + 1 < F::NRB / G; p += 2)
@@ -416,8 +505,10 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
                                 Two o0, o1;
                                 butterfly(y[p * G + x], y[(p + 1) * G + x], L, lane, o0, o1);
                                 const int m = m0 + p * 2 * G + 2 * L;
-                                emit(m, o0);
-                                emit(m + 1, o1);
+                                if (live) {
+                                    emit(m, o0);
+                                    emit(m + 1, o1);
+                                }
                             }
                         }
                 }
@@ -433,7 +524,7 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
                     y[e + G] = o1;
                 }
             if constexpr (STAGE2) {
-                if (nb > 0) {                 // even bands: the pass's outputs
+                if (nb > 0 && live) {                    // even bands: the pass's outputs
                     const int m0 = fresh(a.mband[r + 1]);
 #pragma unroll
                     for (int g = 0; g < F::NRB / (2 * G); g++)
@@ -450,67 +541,67 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
             }
         }
         if constexpr (!STAGE2) {
-            // Ring positions are multiples of 64 when the chunk is, so that a tile never wraps;
-            // with half tiles they are multiples of 32 and the test is made per lane (a lane's
-            // two samples never part).
-            const int q = roff + rpos;
+            // Ring positions and capacities are multiples of 32: a lane's two samples never
+            // part. The lane reads stay outside the branch on live: what is formed inside it is
+            // formed for live lanes only, and lane 0 is not one.
+            if (!__any(rpos + nv > rcap)) {
+                const int q = roff + rpos;
 #pragma unroll
-            for (int hp = 0; hp < F::NRB; hp++) {
-                if constexpr (HC) {
-                    const int cap = __builtin_amdgcn_readlane(rcap, hp);
-                    int x = __builtin_amdgcn_readlane(rpos, hp) + 2 * lane - F::OV;
-                    x -= (x >= cap) ? cap : 0;
-                    if (live)
-                        st2_st(dst + (long(__builtin_amdgcn_readlane(roff, hp)) + x), y[hp].x, y[hp].y);
-                } else {
+                for (int hp = 0; hp < F::NRB; hp++) {
                     Tst *row = dst + (long(__builtin_amdgcn_readlane(q, hp)) - F::OV);
                     if (live)
                         st2_st(row + unsigned(2 * lane), y[hp].x, y[hp].y);
                 }
+            } else {
+#pragma unroll
+                for (int hp = 0; hp < F::NRB; hp++) {
+                    const int cap = __builtin_amdgcn_readlane(rcap, hp);
+                    Tst *row = dst + long(__builtin_amdgcn_readlane(roff, hp));
+                    int q = __builtin_amdgcn_readlane(rpos, hp) + 2 * lane - F::OV;
+                    q -= (q >= cap) ? cap : 0;
+                    if (live)
+                        st2_st(row + q, y[hp].x, y[hp].y);
+                }
             }
-            advance(SH);
+            advance(nv);
         }
         __syncthreads();
     };
 
-    if ((start + 1) * 64 <= a.Tp)
-        load_a(start * 64, Full{});
-    else if (HC)
-        load_a(start * 64, Half{});
-    const int nfull = a.Tp >> 6;
+    load_a(start * U);
+    const int nfull = a.Tp / U;
     for (int it = start; it < min(end, nfull); it++)
-        tile_step(it * 64, it < first, Full{});
-    if constexpr (HC) {
-        if (end > nfull)
-            tile_step(nfull * 64, false, Half{});
-    }
+        tile_step(it * U, it < first, Full{});
+    if (end > nfull)
+        tile_step(nfull * U, false, a.Tp - nfull * U);
 
     if (blockIdx.z + 1 == gridDim.z) {
-        const int hi = (HC && (a.Tp & 63)) ? (a.Tp & 63) : 64;
+        if constexpr (F::HIST) {
 #pragma unroll
-        for (int s = 0; s < F::SA; s++)
-            save_hist<F::K1>(ha[s], wr + (wid + s * F::NW) * SA_::NST, lane, hi);
+            for (int s = 0; s < F::SA; s++)
+                save_hist<F::K1>(ha[s], wr + F::NRES + (wid + s * F::NW) * SA_::NST, lane, (a.Tp - 1) % U + 1);
+        }
         for (int h = 0; h < F::NRB; h++) {
             const float *p = lbuf + line0 + F::line(h, bj);
-            float *r = wr + F::NRB * SA_::NST + F::res(h, j, bj, sumb);
+            float *r = wr + F::res(h, j, bj, sumb);
             for (int q = lane; q < F::lag(h, bj) + F::OV; q += 64)
                 r[q] = p[q];
         }
     }
 }
 
-template<typename Tst, int DD, bool HC>
+template<typename Tst, int DD>
 __global__ void __launch_bounds__(RegDims<DD>::NW * 64) __attribute__((amdgpu_waves_per_eu((DD >= 4) ? 4 : 2)))
 k_stage1(Stage1Args a)
 {
-    reg_tree_body<Tst, DD, false, HC>(a);
+    reg_tree_body<Tst, DD, false>(a);
 }
 
-template<typename Tst, int DD, bool HC>
+template<typename Tst, int DD>
 __global__ void __launch_bounds__(RegDims<DD>::NW * 64) __attribute__((amdgpu_waves_per_eu((DD >= 4) ? 4 : 2)))
 k_stage2(Stage2Args a)
 {
-    reg_tree_body<Tst, DD, true, HC>(a);
+    reg_tree_body<Tst, DD, true>(a);
 }
 
 }  // namespace
@@ -549,7 +640,7 @@ static int tree_nseg(long ninst, int Tp)
     using F = RegDims<DD>;
     constexpr int kStart = 2;
     constexpr long slots = 256L * cmin(16 / F::NW, 160 * 1024 / F::LDS_BYTES);
-    const int ntiles = (Tp + 63) >> 6;
+    const int ntiles = (Tp + F::U - 1) / F::U;
     int best = 1;
     long cost = 0;
     for (int n = 1; n == 1 || (ntiles / n >= cmin(F::WARM, ntiles) && n <= ntiles); n *= 2) {
@@ -564,12 +655,11 @@ static int tree_nseg(long ninst, int Tp)
 }
 
 template<int DD, typename Args>
-static void launch_tree(void (*full)(Args), void (*half)(Args), const Args &a0, hipStream_t st)
+static void launch_tree(void (*k)(Args), const Args &a0, hipStream_t st)
 {
     using F = RegDims<DD>;
     Args a = a0;
     a.nseg = tree_nseg<DD>((1L << a.amb) * a.B, a.Tp);
-    auto *k = (a.Tp & 63) ? half : full;
     allow_lds((const void *) k, F::LDS_BYTES);
     hipLaunchKernelGGL(k, dim3(1 << a.amb, a.B, a.nseg), dim3(F::NW * 64), F::LDS_BYTES, st, a);
 }
@@ -578,7 +668,7 @@ template<typename Tst>
 static void launch_stage1_t(const Stage1Args &a, hipStream_t st)
 {
     switch (a.dd) {
-#define PDD_T(DDV) case DDV: launch_tree<DDV>(k_stage1<Tst, DDV, false>, k_stage1<Tst, DDV, true>, a, st); break;
+#define PDD_T(DDV) case DDV: launch_tree<DDV>(k_stage1<Tst, DDV>, a, st); break;
         PDD_T(1) PDD_T(2) PDD_T(3) PDD_T(4) PDD_T(5) PDD_T(6) PDD_T(7) PDD_T(8)
 #undef PDD_T
         default: break;
@@ -589,7 +679,7 @@ template<typename Tst>
 static void launch_stage2_t(const Stage2Args &a, hipStream_t st)
 {
     switch (a.dd) {
-#define PDD_T(DDV) case DDV: launch_tree<DDV>(k_stage2<Tst, DDV, false>, k_stage2<Tst, DDV, true>, a, st); break;
+#define PDD_T(DDV) case DDV: launch_tree<DDV>(k_stage2<Tst, DDV>, a, st); break;
         PDD_T(1) PDD_T(2) PDD_T(3) PDD_T(4) PDD_T(5) PDD_T(6) PDD_T(7) PDD_T(8)
 #undef PDD_T
         default: break;

@@ -80,6 +80,9 @@ struct Stage2Args {
 // State per tree instance and chunk parity: tree_state_nelts(dd) floats. state_bstride holds two
 // parities: [parity][2^amb instances].
 long tree_state_nelts(int dd);
+// Stage 2 reads a ring row from up to this many samples before the chunk's delayed start (phase
+// A's window).
+static constexpr int kTreeOverlap = 8;
 void launch_stage1(Dtype dt, const Stage1Args &a, hipStream_t st);
 void launch_stage2(Dtype dt, const Stage2Args &a, hipStream_t st);
 
