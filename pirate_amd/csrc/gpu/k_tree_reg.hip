@@ -179,12 +179,17 @@ __device__ __forceinline__ int fresh(int x)
 // Reads the windows at the start of the lines of rows h0 .. h0 + NL - 1 of a phase-B sub-tree
 // and moves these lines down by sh samples (U, or the chunk's last samples: even). All by one
 // wave, whose LDS instructions execute in order; a line's loads are issued before the stores that
-// may overwrite what they read, and the loads of NL lines are in flight together.
+// may overwrite what they read, and the loads of NL lines are in flight together. Of every line
+// the first lag(h0) + OV samples are stored, under one mask: the lag falls with h, and what that
+// writes past a line's own lag + OV samples lies in its tile, which phase A writes next.
 template<int DD, int NL, bool READ>
 __device__ __forceinline__ void take_lines(float *lj, int h0, int b, int lane, int sh, Two *v)
 {
     using F = RegDims<DD>;
+    static_assert((NL - 1) * (F::NRA - 1) <= F::U, "lag(h0) + OV samples of a line lie within it");
+    const int keep = F::lag(h0, b) + F::OV;
     constexpr bool LONG = F::LMAX + F::OV > 128;
+    const bool lng = LONG && keep > 128;      // wave-uniform
     float2 s0[NL], s1[NL];
 #pragma unroll
     for (int i = 0; i < NL; i++) {
@@ -195,20 +200,22 @@ __device__ __forceinline__ void take_lines(float *lj, int h0, int b, int lane, i
             v[i].y = w.y;
         }
         s0[i] = q[sh / 2];
-        if constexpr (LONG)
-            if (F::lag(h0 + i, b) + F::OV > 128)      // wave-uniform
-                s1[i] = q[sh / 2 + 64];
+    }
+    if (lng) {
+#pragma unroll
+        for (int i = 0; i < NL; i++)
+            s1[i] = reinterpret_cast<const float2 *>(lj + F::line(h0 + i, b))[lane + sh / 2 + 64];
     }
     __builtin_amdgcn_wave_barrier();
+    if (2 * lane < keep) {
 #pragma unroll
-    for (int i = 0; i < NL; i++) {
-        float2 *q = reinterpret_cast<float2 *>(lj + F::line(h0 + i, b)) + lane;
-        const int keep = F::lag(h0 + i, b) + F::OV;
-        if (2 * lane < keep)
-            q[0] = s0[i];
-        if constexpr (LONG)
-            if (128 + 2 * lane < keep)
-                q[64] = s1[i];
+        for (int i = 0; i < NL; i++)
+            reinterpret_cast<float2 *>(lj + F::line(h0 + i, b))[lane] = s0[i];
+    }
+    if (lng && 128 + 2 * lane < keep) {
+#pragma unroll
+        for (int i = 0; i < NL; i++)
+            reinterpret_cast<float2 *>(lj + F::line(h0 + i, b))[lane + 64] = s1[i];
     }
     __builtin_amdgcn_wave_barrier();
 }
@@ -546,11 +553,14 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
             // formed for live lanes only, and lane 0 is not one.
             if (!__any(rpos + nv > rcap)) {
                 const int q = roff + rpos;
+                int qs[F::NRB];
 #pragma unroll
-                for (int hp = 0; hp < F::NRB; hp++) {
-                    Tst *row = dst + (long(__builtin_amdgcn_readlane(q, hp)) - F::OV);
-                    if (live)
-                        st2_st(row + unsigned(2 * lane), y[hp].x, y[hp].y);
+                for (int hp = 0; hp < F::NRB; hp++)
+                    qs[hp] = __builtin_amdgcn_readlane(q, hp);
+                if (live) {
+#pragma unroll
+                    for (int hp = 0; hp < F::NRB; hp++)
+                        st2_st(dst + (long(qs[hp]) - F::OV) + unsigned(2 * lane), y[hp].x, y[hp].y);
                 }
             } else {
 #pragma unroll
