@@ -40,11 +40,11 @@
 // stay inside the chunk, its stores stop at the chunk's end, and the lines move down by its
 // length.
 //
-// Bounded by VALU issue (about 65% busy in float16) and the round trips of a tile (row loads,
-// two barriers, LDS lines), not by bytes: rank 7 runs at 4.2-4.6 TB/s in float32, 2.8-3.0 in
+// Bounded by the round trips of a tile (row loads, two barriers, LDS lines; waves wait half of
+// their time), then by VALU issue (62% busy in float16), not by bytes: rank 7 runs at 4.2-4.6 TB/s in float32, 2.9-3.2 in
 // float16. 16 beams of 16384 channels x 2048 samples, stages 1 and 2 (rank 7): float16 0.83 and
-// 0.86 ms with tiles of 64 and phase-A histories, 0.72 and 0.77 ms now; float32 0.99 and 0.95,
-// 1.01 and 0.94 ms. Rank 8 (4 beams of 65536 channels, float16) with histories 1.05 and 1.08 ms,
+// 0.86 ms with tiles of 64 and phase-A histories, 0.69 and 0.75 ms now; float32 0.99 and 0.95,
+// 1.00 and 0.90 ms. Rank 8 (4 beams of 65536 channels, float16) with histories 1.05 and 1.08 ms,
 // in windows and tiles of 64 1.16 and 1.26, of 80 1.07 and 1.14; its subband stage 2 1.26, 1.48
 // and 1.61 ms (rows of 80 16-bit samples start inside 64-byte blocks).
 // No kernel spills, and none calls a function: with the line offsets in a recursive constexpr
@@ -190,32 +190,32 @@ __device__ __forceinline__ void take_lines(float *lj, int h0, int b, int lane, i
     const int keep = F::lag(h0, b) + F::OV;
     constexpr bool LONG = F::LMAX + F::OV > 128;
     const bool lng = LONG && keep > 128;      // wave-uniform
-    float2 s0[NL], s1[NL];
+    float2 s0[NL], s1[NL], *q[NL];
 #pragma unroll
     for (int i = 0; i < NL; i++) {
-        const float2 *q = reinterpret_cast<const float2 *>(lj + F::line(h0 + i, b)) + lane;
+        q[i] = reinterpret_cast<float2 *>(lj + fresh(F::line(h0 + i, b))) + lane;
         if constexpr (READ) {
-            const float2 w = *q;
+            const float2 w = *q[i];
             v[i].x = w.x;
             v[i].y = w.y;
         }
-        s0[i] = q[sh / 2];
+        s0[i] = q[i][sh / 2];
     }
     if (lng) {
 #pragma unroll
         for (int i = 0; i < NL; i++)
-            s1[i] = reinterpret_cast<const float2 *>(lj + F::line(h0 + i, b))[lane + sh / 2 + 64];
+            s1[i] = q[i][sh / 2 + 64];
     }
     __builtin_amdgcn_wave_barrier();
     if (2 * lane < keep) {
 #pragma unroll
         for (int i = 0; i < NL; i++)
-            reinterpret_cast<float2 *>(lj + F::line(h0 + i, b))[lane] = s0[i];
+            *q[i] = s0[i];
     }
     if (lng && 128 + 2 * lane < keep) {
 #pragma unroll
         for (int i = 0; i < NL; i++)
-            reinterpret_cast<float2 *>(lj + F::line(h0 + i, b))[lane + 64] = s1[i];
+            q[i][64] = s1[i];
     }
     __builtin_amdgcn_wave_barrier();
 }
@@ -365,26 +365,41 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
             }
         } else {
             const unsigned tb = unsigned(i) * unsigned(sizeof(Tst));
-            if (!__any(rpos + wlen > rcap)) {
-                const int q = roff + rpos;
+            const int q = roff + rpos;
+            const unsigned long long wrap = __ballot(rpos + wlen > rcap);
+            auto load_row = [&](int s, int l) {
+                const Tst *row = src + long(__builtin_amdgcn_readlane(q, s * F::NRA + l));
+                xa[s][l].load(reinterpret_cast<const Tst *>(reinterpret_cast<const char *>(row) + tb));
+            };
+            if (wrap == 0) {
 #pragma unroll
                 for (int s = 0; s < F::SA; s++)
 #pragma unroll
-                    for (int l = 0; l < F::NRA; l++) {
-                        const Tst *row = src + long(__builtin_amdgcn_readlane(q, s * F::NRA + l));
-                        xa[s][l].load(reinterpret_cast<const Tst *>(reinterpret_cast<const char *>(row) + tb));
-                    }
+                    for (int l = 0; l < F::NRA; l++)
+                        load_row(s, l);
             } else {
+                // About one tile in two: some row wraps. Float32 loads only such rows sample by
+                // sample (stage 2 0.933 -> 0.904 ms); 16-bit types do it for all rows, since
+                // with both ways the halves of a pair make the compiler wait row by row
+                // (0.752 -> 0.939 ms), and so does rank 8, for want of registers.
+                constexpr bool ALL = sizeof(Tst) == 2 || F::S == 1;
 #pragma unroll
                 for (int s = 0; s < F::SA; s++)
 #pragma unroll
                     for (int l = 0; l < F::NRA; l++) {
-                        const int k = s * F::NRA + l, cap = __builtin_amdgcn_readlane(rcap, k);
-                        const Tst *row = src + long(__builtin_amdgcn_readlane(roff, k));
-                        const int q0 = __builtin_amdgcn_readlane(rpos, k) + i, q1 = q0 + 1;
-                        xa[s][l].set(row + (q0 - ((q0 >= cap) ? cap : 0)), row + (q1 - ((q1 >= cap) ? cap : 0)));
+                        const int k = s * F::NRA + l;
+                        if (ALL || ((wrap >> k) & 1)) {
+                            const int cap = __builtin_amdgcn_readlane(rcap, k);
+                            const Tst *row = src + long(__builtin_amdgcn_readlane(roff, k));
+                            const int q0 = __builtin_amdgcn_readlane(rpos, k) + i, q1 = q0 + 1;
+                            xa[s][l].set(row + (q0 - ((q0 >= cap) ? cap : 0)), row + (q1 - ((q1 >= cap) ? cap : 0)));
+                            if constexpr (!ALL)
+                                asm volatile("");        // keeps the branches' loads (and their addresses) apart
+                        } else {
+                            load_row(s, l);
+                        }
                     }
-                asm volatile("");        // keeps the two branches' loads (and their addresses) apart
+                asm volatile("");
             }
             advance(U);
         }
@@ -448,7 +463,7 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
                     for (int jj = 0; jj < F::NRA; jj++) {
                         constexpr int K1 = F::K1;
                         const int b1 = brev_c(jj, K1);
-                        float *p = lbuf + (F::CQ.v[jj] + F::line(h, b1) + F::lag(h, b1) + F::OV - F::OVA) + 2 * lane;
+                        float *p = lbuf + fresh(F::CQ.v[jj] + F::line(h, b1) + F::lag(h, b1) + F::OV - F::OVA) + 2 * lane;
                         p[0] = x[jj].x;
                         p[1] = x[jj].y;
                     }
@@ -632,7 +647,7 @@ long tree_state_nelts(int dd)
     }
 }
 
-// Dynamic LDS above 64 KB (rank 8) must be allowed per kernel; gfx950 allows 160 KB.
+// Dynamic LDS above 64 KB (ranks 7 and 8) must be allowed per kernel; gfx950 allows 160 KB.
 static void allow_lds(const void *fn, int bytes)
 {
     if (bytes > 65536)
@@ -642,7 +657,7 @@ static void allow_lds(const void *fn, int bytes)
 // Time segments: a segment of n tiles runs n + WARM; workgroups run in rounds of as many as fit
 // on the chip (256 CUs, 16 waves and 160 KB of LDS each), and a round costs about kStart tiles
 // besides (launch, state). Takes the power of two with the shortest sum. One beam of rank 10
-// (32 instances x 32 tiles): 16 segments, stages 1 and 2 54 and 64 us -> 12 and 12 us; from some
+// (32 instances x 22 tiles): stages 1 and 2 54 and 64 us in one segment, 13 and 12 us in 16; from some
 // 500 instances on, one segment.
 template<int DD>
 static int tree_nseg(long ninst, int Tp)
