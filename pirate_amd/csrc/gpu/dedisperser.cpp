@@ -1166,8 +1166,8 @@ void GpuDedisperser::tree_rows(long itree, void *&base, long &nrows, long &beam_
     nrows = long(t.ndm_out) * T.M;
     row_stride = T.rowlen;
     beam_stride = nrows * T.rowlen;
-    // the peak finder ends the chunk by moving its last tpad + flmax samples to the row
-    // start, so [flmax, nt_ds) is what still holds this chunk's samples
+    // the peak finder ends the chunk by copying its last tpad samples to the row's history, so all
+    // of the chunk is there; t_lo, the largest final lag, is where callers start to read
     t_lo = T.flmax;
     t_hi = t.nt_ds;
 }

@@ -135,8 +135,8 @@ public:
     size_t debug_copy(const std::string &name, void *host, size_t maxbytes);
     // Peak-finder input rows of tree itree (the stage-2 output): row r = idm_out * M + m of global
     // beam b, chunk sample t at base + (b * beam_stride + r * row_stride + t) * elt_bytes. After
-    // the chunk's peak finding (i.e. once its output is acquired) samples flmax <= t < nt_ds of
-    // the latest chunk of the beam's batch are there (flmax = 0 without subband final lags).
+    // the chunk's peak finding (i.e. once its output is acquired) samples t_lo <= t < t_hi of
+    // the latest chunk of the beam's batch are there (t_lo: the largest subband final lag, else 0).
     void tree_rows(long itree, void *&base, long &nrows, long &beam_stride, long &row_stride, long &t_lo,
                    long &t_hi);
 

@@ -509,8 +509,8 @@ k_pf_var(PfArgs a)
 // neighbouring rows cover all banks. 49 KB of LDS and 168 VGPRs: three workgroups (12 waves)
 // per CU. Bounded by VALU issue (about 400 instructions per stream and 16-sample bin at Wmax 16,
 // against 520 with every candidate compared) and, for float32, near half by the row reads.
-// 16384 DM rows x 2048 samples x 16 beams, Wmax 16, bins of 16: float32 0.774 -> 0.558 ms,
-// float16 0.736 -> 0.444 ms; 36 multiplets, 8 beams of rank 15, float16: 2.28 -> 1.19 ms.
+// 16384 DM rows x 2048 samples x 16 beams, Wmax 16, bins of 16: float32 0.774 -> 0.547 ms,
+// float16 0.736 -> 0.422 ms; 36 multiplets, 8 beams of rank 15, float16: 2.28 -> 1.01 ms.
 // Tried: tiles of 16 positions staged through registers (each 128-byte line fetched twice,
 // float32 0.93 ms), two staging buffers and 8 waves per CU (0.68 ms), the walk's float32 loads
 // all at once with bins of 16 (31 registers spilled, 1.31 ms).
