@@ -38,7 +38,7 @@ def _is_lib(name):
 
 
 def _short(name):
-    s = name.replace('void ', '').replace(LIB_PREFIX, '')
+    s = name.replace('void ', '').replace(LIB_PREFIX, '').replace('(anonymous namespace)::', '')
     return s.split('(')[0]
 
 
