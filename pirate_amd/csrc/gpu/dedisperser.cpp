@@ -295,7 +295,8 @@ void GpuDedisperser::allocate()
                 long r = a1 * pow2(dd1) + j;
                 if (minlag >= 0 && max_gpu_clag < (1L << 40))
                     kr[r] = std::max(0L, minlag / Tp - max_gpu_clag);
-                cap[r] = align_up(maxlag - kr[r] * Tp + Tp + kTreeOverlap, 64);
+                // rows of whole 128-byte lines (16-bit rows of 64 bytes: stages 1 and 2 1 to 2% slower)
+                cap[r] = align_up(maxlag - kr[r] * Tp + Tp + kTreeOverlap, 128 / elt_bytes);
                 off[r] = tot;
                 tot += cap[r];
             }
