@@ -231,12 +231,13 @@ struct PfLane {
 
 // The same walk without weights or codes: the largest value of every profile in a bin (the
 // weight of a profile is constant over a bin, and rounding is monotonic, so the largest
-// weighted candidate of a profile is its weight times this value, bit for bit).
+// weighted candidate of a profile is its weight times this value, bit for bit). That needs
+// finite values: a candidate that is not finite can be NaN once weighted, and PfLane drops a level
+// whose first candidate is NaN (a zero weight times -inf, say), which no maximum shows.
 template<typename S>
 struct PfMax {
     float w[S::WTOT];          // boxcar windows, as in PfLane
     float mx[S::P];            // per profile: largest value in the current bin
-    bool nonfinite;            // an infinity or NaN entered the windows in the current bin
 
     template<int L, int POS, bool EVAL>
     __device__ __forceinline__ void levels()
@@ -251,8 +252,6 @@ struct PfMax {
                         w[o + i] = w[o + i - 1];
                     w[o] = w[op + back] + w[op];
                 }
-                if constexpr (L == S::NLEV - 1)        // every sample enters one of these sums
-                    nonfinite |= !(fabsf(w[o]) < __builtin_inff());
                 if constexpr (EVAL) {
                     constexpr bool first = (POS + 1) / S::dt(L) == 1;
                     const float x3 = w[o], x2 = w[o + s], x1 = w[o + 2 * s], x0 = w[o + 3 * s];
@@ -287,18 +286,13 @@ struct PfMax {
         }
     }
 
-    // The bin's largest weighted value V, the first level that has it, and whether a weighted
-    // maximum is NaN (an infinite value times a zero weight).
-    __device__ __forceinline__ bool combine(const float (&wt)[S::P], float &V, unsigned int &lev) const
+    // The bin's largest weighted value V and the first level that has it.
+    __device__ __forceinline__ void combine(const float (&wt)[S::P], float &V, unsigned int &lev) const
     {
         float v[S::P];
 #pragma unroll
         for (int p = 0; p < S::P; p++)
             v[p] = wt[p] * mx[p];
-        bool nan = false;
-#pragma unroll
-        for (int p = 0; p < S::P; p += 2)
-            nan |= __builtin_isunordered(v[p], v[(p + 1 < S::P) ? p + 1 : p]);
         V = v[0];
         lev = 0;
         if constexpr (S::P > 1) {
@@ -310,9 +304,22 @@ struct PfMax {
                 V = fmaxf(V, u);
             }
         }
-        return nan;
     }
 };
+
+// Whether a bin's samples are such that PfMax may not be used for it, nor for the NBACK bins after
+// it, whose windows they enter: a candidate adds at most 64 samples (times up to 1), so with
+// samples below 1e36 all candidates are finite. One three-operand maximum, which keeps NaN, for
+// two samples.
+template<int N>
+__device__ __forceinline__ bool pf_wild(const float *x)
+{
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; i++)
+        m = __builtin_elementwise_maximum(m, fabsf(x[i]));
+    return !(m < 1e36f);
+}
 
 __device__ __forceinline__ int pf_level_of_token(unsigned int tok)
 {
@@ -497,8 +504,8 @@ k_pf_var(PfArgs a)
 // it picks the winning multiplet (largest value, then first (level, m)) and walks that one
 // stream over the bin again with PfLane, which gives the value and the token of the first
 // maximum. A DM row has M streams, so step 2 costs 1/M of a full walk per stream.
-// Infinities and NaN: a stream whose windows held one, or whose weighted maxima hold a NaN, is
-// marked, and step 2 walks every stream of a marked (DM row, bin) with PfLane.
+// Infinities, NaN and samples that could make a sum overflow (pf_wild): a stream is marked in each
+// bin whose windows hold one, and step 2 walks every stream of a marked (DM row, bin) with PfLane.
 //
 // Samples reach LDS by direct loads (no registers, no conversion), 128 bytes of a row at a
 // time, so that every line is fetched once; a wave stages the 64 rows that its lanes walk, so
@@ -564,7 +571,7 @@ k_pf(PfArgs a)
 #pragma unroll
     for (int i = 0; i < S::WTOT; i++)
         ln.w[i] = 0.0f;
-    int marked = 0;            // bins, from this one on, whose windows hold an infinity or NaN
+    int marked = 0;            // bins, from this one on, whose windows hold a sample that pf_wild rejects
 
     // The first tile holds the line of position tpad - 1: nwarm tiles reach back to the line of
     // position 0 (rows start 'lead' elements after a line; what lies before position 0 in
@@ -612,10 +619,8 @@ k_pf(PfArgs a)
             if (it < nwarm) {
 #pragma unroll
                 for (int j = 0; j < BPS; j++) {
-                    ln.nonfinite = false;
+                    marked = pf_wild<S::DOUT>(x + j * S::DOUT) ? NBACK + 1 : max(marked - 1, 0);
                     ln.template bin<false>(x + j * S::DOUT);
-                    marked = ln.nonfinite ? NBACK + 1 : marked;
-                    marked = max(marked - 1, 0);
                 }
                 continue;
             }
@@ -630,15 +635,13 @@ k_pf(PfArgs a)
 #pragma unroll
                     for (int p = 0; p < S::P; p++)
                         wt[p] = wp[p * N];
-                    ln.nonfinite = false;
+                    marked = pf_wild<S::DOUT>(x + j * S::DOUT) ? NBACK + 1 : max(marked - 1, 0);
                     ln.template bin<true>(x + j * S::DOUT);
                     float V;
                     unsigned int lev;
-                    const bool nan = ln.combine(wt, V, lev);
-                    marked = ln.nonfinite ? NBACK + 1 : marked;
+                    ln.combine(wt, V, lev);
                     rv[(nbatch + j) * RVS + tid] = V;
-                    rl[(nbatch + j) * RLS + tid] = (unsigned char)((marked > 0 || nan) ? 0x80u : lev);
-                    marked = max(marked - 1, 0);
+                    rl[(nbatch + j) * RLS + tid] = (unsigned char)((marked > 0) ? 0x80u : lev);
                 }
             }
             nbatch += BPS;

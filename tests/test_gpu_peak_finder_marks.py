@@ -1,0 +1,83 @@
+"""The two-step peak finder where values leave the range in which its first step is exact, bit for
+bit against the kernel that visits every candidate in order (the one that also forms the float64
+variances): boxcar sums of finite samples that overflow, with zero weights on some profiles."""
+
+import numpy as np
+import pytest
+
+from gpu_cases import BASE, pt
+from gpu_harness import random_weights
+
+pytestmark = pytest.mark.gpu
+
+
+def make_pair(rank, bands, widths, dtype, B, T, time_ds=0):
+    """The same search with the peak finder proper and with the one that forms variances."""
+    import pirate_amd as pa
+    trees = [dict(pt(0, w, min(64, 2**(rank - 1)), 64), time_downsampling=time_ds) for w in widths]
+    cfg = dict(BASE, dtype=dtype, zone_nfreq=[2**rank], zone_freq_edges=[400, 800], toplevel_tree_rank=rank,
+               time_samples_per_chunk=T, beams_per_gpu=B, beams_per_batch=B, num_active_batches=1,
+               frequency_subband_counts=bands, primary_trees=trees)
+    plan = pa.DedispersionPlan(pa.DedispersionConfig.from_dict(cfg))
+    dds = [pa.GpuDedisperser(plan, enable_variances=v) for v in (False, True)]
+    rng = np.random.default_rng(rank)
+    for dd in dds:
+        dd.allocate()
+    for it in range(plan.ntrees):
+        w = random_weights(rng, dds[0], it)
+        for dd in dds:
+            dd.fill_all_weights(it, w)
+    return plan, dds
+
+
+def outputs(plan, dds, c, x):
+    """Bit patterns of (out_max, out_argmax) of every tree, for each of the two."""
+    import torch
+    x = torch.from_numpy(x).cuda()
+    bits = torch.int32 if plan.dtype == 'float32' else torch.int16
+    res = []
+    for dd in dds:
+        with dd.get_input(c) as arr:
+            arr.copy_(x)
+        with dd.get_output(c) as out:
+            res.append([(m.view(bits).cpu().numpy(), a.cpu().numpy(), m.float().cpu().numpy())
+                        for m, a in zip(out.out_max, out.out_argmax)])
+    return res
+
+
+def assert_equal(plan, res, c):
+    for it in range(plan.ntrees):
+        for i, what in enumerate(('out_max', 'out_argmax')):
+            a, b = res[0][it][i], res[1][it][i]
+            assert np.array_equal(a, b), f'chunk {c} tree {it} {what}: {int(np.sum(a != b))} of {a.size} differ'
+
+
+# bins of 16, 8 and 16 samples; 16, 34 and 91 multiplets
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('rank,bands', [(13, [0, 0, 0, 0, 1]), (11, [4, 5, 3, 1]), (14, [5, 9, 7, 3, 1])])
+def test_sums_that_overflow(rank, bands, dtype):
+    """Pairs of neighbouring samples of -1.72e38 at zero DM on a small positive background, each pair
+    on both sides of a bin's start: their sum is -inf, while all sums on the boxcar levels' grids (and of the
+    other multiplets, which smear a pair over more samples) are finite. Such a sum is then the first candidate of its level, and times a zero weight NaN: the level
+    is out for this bin and stream, whatever its later candidates are. Weights are zero but for the second and
+    third profile of one level."""
+    B, T = 2, 512
+    print(f'[peak finder marks] overflow rank {rank} {bands} {dtype}', flush=True)
+    plan, dds = make_pair(rank, bands, [16], dtype, B, T)
+    bin_len = T // plan.trees[0].nt_out
+    rng = np.random.default_rng(1)
+    w = np.zeros(dds[0].wt_shape(0), dtype=np.float32)          # (slots, B, ndm_wt, nt_wt, P, N)
+    lev = rng.integers(1, 4, size=w.shape[:4] + w.shape[5:])
+    for l in (1, 2, 3):
+        for p in (3 * l + 2, 3 * l + 3):
+            w[:, :, :, :, p, :] = (lev == l) * rng.uniform(0.5, 1, size=lev.shape)
+    for dd in dds:
+        dd.fill_all_weights(0, w)
+    for c in range(3):
+        v = 1e30 * (1 + 0.3 * rng.standard_normal((B, plan.nfreq, T)))
+        for b in range(B):
+            for k in rng.choice(np.arange(1, T // bin_len), T // bin_len // 3, replace=False):
+                v[b, :, k * bin_len - 1:k * bin_len + 1] = -1.72e38
+        x = (v * 2.0 ** (-rank / 2)).astype(np.float32)
+        res = outputs(plan, dds, c, x)
+        assert_equal(plan, res, c)
