@@ -237,8 +237,9 @@ int pdd_dedisperser_spill_bytes(const pdd_dedisperser *dd, int64_t *nbytes);
 
 /* Launch shapes that change no output, only speed (no reference counterpart: the reference
  * fixes its launch shapes in its kernel generators). name: "pf_target_blocks" (the peak
- * finder splits each chunk into the fewest power-of-two time segments giving at least this
- * many workgroups; default 2048), "grid_xcd_run" (gridding workgroups per XCD run of adjacent
+ * finder splits each chunk into at most the fewest time segments giving at least this many
+ * workgroups; default 2048), "pf_two_step" (the peak finder's two-step kernel: automatic = -1,
+ * never = 0, wherever there is one = 1), "grid_xcd_run" (gridding workgroups per XCD run of adjacent
  * channel pairs; 0 = launch order; default 8), "fork" (primary trees p >= 1 start after the
  * gridding = 0, after tree 0's stage 2 = 1, automatic = -1, all kernels in order on one stream
  * = 2, for per-kernel timing). Takes effect at the next launch. */

@@ -4,9 +4,9 @@
                                   [--out pirate_amd/tuning_table.json] [--steps 10]
 
 The launch shapes change no output, only speed (GpuDedisperser.set_tuning):
-  * pf_target_blocks: the peak finder splits each chunk's time axis into the fewest segments
-    (one work group each, warmed up over the history samples) that give at least this many
-    work groups;
+  * pf_target_blocks: the peak finder splits each chunk's time axis into at most the fewest
+    segments (one work group each, warmed up over the history samples) that give at least this
+    many work groups;
   * grid_xcd_run: consecutive channel pairs that the fused gridding kernel gives each of the 8
     XCDs (0: plain launch order), which sets how the input rows of neighbouring tree channels
     share an XCD's L2;

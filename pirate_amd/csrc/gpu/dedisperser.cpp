@@ -453,6 +453,10 @@ void GpuDedisperser::set_tuning(const std::string &name, long value)
         PDD_CHECK(value >= 1 && value <= (1L << 20), "set_tuning(): pf_target_blocks must be in [1, 2^20]");
         tuning.pf_target_blocks = value;
     }
+    else if (name == "pf_two_step") {
+        PDD_CHECK(value >= -1 && value <= 1, "set_tuning(): pf_two_step must be -1, 0 or 1");
+        tuning.pf_two_step = int(value);
+    }
     else if (name == "grid_xcd_run") {
         PDD_CHECK(value >= 0 && value <= 64, "set_tuning(): grid_xcd_run must be in [0, 64]");
         tuning.grid_xcd_run = int(value);
@@ -469,6 +473,8 @@ long GpuDedisperser::get_tuning(const std::string &name) const
 {
     if (name == "pf_target_blocks")
         return tuning.pf_target_blocks;
+    if (name == "pf_two_step")
+        return tuning.pf_two_step;
     if (name == "grid_xcd_run")
         return tuning.grid_xcd_run;
     if (name == "fork")
@@ -672,6 +678,7 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
             f.nt_out = int(t.nt_out);
             f.beam0 = beam0;
             f.target_blocks = tuning.pf_target_blocks;
+            f.two_step = tuning.pf_two_step;
             if (params.enable_variances)
                 f.out_var = (double *) out_var[it].ptr + oslot * B * t.ndm_out * T.M * t.nprofiles;
             const std::string nmp = "pf_t" + std::to_string(it);

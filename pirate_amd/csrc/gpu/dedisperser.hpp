@@ -36,7 +36,8 @@ struct GpuDedisperserParams {
 // Launch shapes that change no result (only speed), settable between chunks; the values
 // below are the defaults, the autotuner's table overrides them per workload.
 struct LaunchTuning {
-    long pf_target_blocks = 2048;   // peak finder: fewest time segments giving this many workgroups
+    long pf_target_blocks = 2048;   // peak finder: at most the fewest time segments giving this many workgroups
+    int pf_two_step = -1;           // peak finder in two steps: -1 auto, 0 never, 1 wherever there is such a kernel
     int grid_xcd_run = 8;           // gridding: consecutive channel pairs per XCD (0: launch order)
     int fork = -1;                  // primary trees p >= 1 start: -1 auto, 0 after the gridding,
                                     // 1 after tree 0's stage 2, 2 serial (no branch streams)
@@ -61,7 +62,7 @@ public:
     // points are then refused (the group launches its chains).
     bool group_member = false;
 
-    // name in {"pf_target_blocks", "grid_xcd_run", "fork"}; throws on a bad name or value.
+    // name in {"pf_target_blocks", "pf_two_step", "grid_xcd_run", "fork"}; throws on a bad name or value.
     void set_tuning(const std::string &name, long value);
     long get_tuning(const std::string &name) const;
 

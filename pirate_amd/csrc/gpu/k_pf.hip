@@ -12,10 +12,10 @@
 // Mapping: one lane per stream (DM row, multiplet m); a block holds 256/M DM rows. Each lane
 // walks its stream through time once. Every boxcar level keeps its last values in a register
 // window (Wmax and Dout are template parameters, so every shift, sum and candidate of one
-// output bin is unrolled at compile time). k_pf keeps the largest value of each profile and
-// finds the token of the winning stream in a second step (below); k_pf_var, which also forms
-// the optional float64 variances, weights and compares each candidate as it is formed (strict
-// '>', candidates visited in (isamp, p) order). Either way the multiplets of a DM row are
+// output bin is unrolled at compile time). k_pf_one weights and compares each candidate as it is
+// formed (strict '>', candidates visited in (isamp, p) order) and can form the optional
+// float64 variances. k_pf keeps the largest value of each profile and finds the token of the
+// winning stream in a second step; pf_two_step says where. Either way the multiplets of a DM row are
 // reduced in (level, m) order, and the result is the reference's maximum and argmax token, bit
 // for bit. Positions before the row start count as zeros, the initial state of the windows.
 //
@@ -33,13 +33,15 @@
 #include "device_common.hpp"
 #include "kernels.hpp"
 
+#include <algorithm>
+
 namespace pirate_amd {
 
 static constexpr int kPfThreads = 256;
 static constexpr int kPfMaxDout = 32;
 static constexpr int kPfLine = 128;      // bytes of a row that one staging tile covers
 
-// k_pf_var's staging tile length (positions) for output time downsampling Dout: whole output
+// k_pf_one's staging tile length (positions) for output time downsampling Dout: whole output
 // bins, at least kPfTileMin positions when Dout >= 4, 8 bins below.
 static constexpr int kPfTileMin = 16;
 __host__ __device__ constexpr int pf_tile_len(int dout)
@@ -72,9 +74,7 @@ struct PfShape {
     static constexpr int win(int l) { return 3 * sgrid(l) + 1; }
     static constexpr int woff(int l) { return (l == 0) ? 0 : woff(l - 1) + win(l - 1); }
     static constexpr int WTOT = woff(NLEV);
-    // Waves per SIMD: 3 (168 VGPRs, as many as the LDS allows) where step 2's unrolled walk
-    // fits, else 2.
-    static constexpr int WAVES = (LD == 5 || (LD == 0 && LW >= 4) || (LD == 1 && LW == 5)) ? 2 : 3;
+    static constexpr int WAVES1 = (WTOT + P <= 32 && LD >= 2) ? 4 : 2;     // k_pf_one's waves per SIMD
 };
 
 template<typename S, bool VAR>
@@ -364,10 +364,14 @@ __device__ __forceinline__ void rotate_rows(Tst *rows, int nstreams, const PfArg
     }
 }
 
-// With the float64 out_var: every candidate is weighted, compared and summed as it is formed.
-template<typename Tst, int LW, int LD>
-__global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
-k_pf_var(PfArgs a)
+// The first evaluated tile of time segment z (of nseg) of a chunk of n tiles.
+__device__ __forceinline__ int pf_first_tile(int n, int z, int nseg) { return int(long(n) * z / nseg); }
+
+// One step: every candidate is weighted and compared as it is formed, and (VAR) its square summed
+// for the float64 out_var.
+template<typename Tst, int LW, int LD, bool VAR>
+__global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(VAR ? 2 : PfShape<LW, LD>::WAVES1)))
+k_pf_one(PfArgs a)
 {
     using S = PfShape<LW, LD>;
     constexpr int TL = S::TL, NB = S::NB, STR = TL + 1, VPR = TL / 4;
@@ -380,8 +384,8 @@ k_pf_var(PfArgs a)
     const int ndpf = kPfThreads / M;
     const int dpf0 = blockIdx.x * ndpf;
     const int b = blockIdx.y;
-    const int ntseg = a.Tp / (TL * a.nseg);      // evaluated tiles of this segment
-    const int tile0 = blockIdx.z * ntseg;        // its first tile in the chunk
+    const int tile0 = pf_first_tile(a.Tp / TL, blockIdx.z, a.nseg);               // this segment's first tile
+    const int ntseg = pf_first_tile(a.Tp / TL, blockIdx.z + 1, a.nseg) - tile0;    // its evaluated tiles
     const int nd = min(ndpf, a.ndm_out - dpf0);
     const int nstreams = nd * M;
     const bool active = tid < nstreams;
@@ -395,16 +399,18 @@ k_pf_var(PfArgs a)
     Tst *outm = reinterpret_cast<Tst *>(a.out_max) + long(b) * a.out_bstride;
     unsigned int *outa = a.out_argmax + long(b) * a.out_bstride;
 
-    PfLane<S, true> ln;
+    PfLane<S, VAR> ln;
 #pragma unroll
     for (int i = 0; i < S::WTOT; i++)
         ln.w[i] = 0.0f;
+    if constexpr (VAR) {
 #pragma unroll
-    for (int p = 0; p < S::P; p++)
-        ln.bs[p] = ln.acc[p] = 0.0;
+        for (int p = 0; p < S::P; p++)
+            ln.bs[p] = ln.acc[p] = 0.0;
 #pragma unroll
-    for (int l = 0; l < S::NLEV; l++)
-        ln.wv[l] = 1.0 / double(a.nt_out * (S::DOUT / S::dt(l)));
+        for (int l = 0; l < S::NLEV; l++)
+            ln.wv[l] = 1.0 / double(a.nt_out * (S::DOUT / S::dt(l)));
+    }
 
     const int nwarm = (a.tpad + TL - 1) / TL;
     const int ntiles = nwarm + ntseg;
@@ -486,7 +492,7 @@ k_pf_var(PfArgs a)
         }
     }
 
-    if (active) {
+    if (VAR && active) {
         double *ov = a.out_var + long(b) * a.ndm_out * M * S::P + (long(dpf0 + dl) * M + m) * S::P;
 #pragma unroll
         for (int p = 0; p < S::P; p++)
@@ -527,7 +533,7 @@ typedef __attribute__((address_space(1))) const void *pf_gptr;
 typedef __attribute__((address_space(3))) void *pf_lptr;
 
 template<typename Tst, int LW, int LD>
-__global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(PfShape<LW, LD>::WAVES)))
+__global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(3)))
 k_pf(PfArgs a)
 {
     using S = PfShape<LW, LD>;
@@ -550,8 +556,8 @@ k_pf(PfArgs a)
     const int ndpf = kPfThreads / M;
     const int dpf0 = blockIdx.x * ndpf;
     const int b = blockIdx.y;
-    const int ntseg = a.Tp / (TL * a.nseg);      // evaluated tiles of this segment
-    const int tile0 = blockIdx.z * ntseg;        // its first tile in the chunk
+    const int tile0 = pf_first_tile(a.Tp / TL, blockIdx.z, a.nseg);               // this segment's first tile
+    const int ntseg = pf_first_tile(a.Tp / TL, blockIdx.z + 1, a.nseg) - tile0;    // its evaluated tiles
     const int nd = min(ndpf, a.ndm_out - dpf0);
     const int nstreams = nd * M;
     const bool active = tid < nstreams;
@@ -691,27 +697,18 @@ k_pf(PfArgs a)
                         pl2.wt[p] = wq[p * N];
                     const Tst *row = rows + long(d * M + mm) * a.rowlen;
                     const int pb = a.tpad + tb * S::DOUT;
-                    // groups of V samples; those before position 0 read as zeros (with DOUT >= 4,
-                    // position 0 starts a group)
-                    constexpr int V = (S::DOUT >= 4) ? 4 : 1, NV = S::DOUT / V;
-                    using Raw = typename std::conditional<V == 4, rawv_st<Tst, 4>, raw_st<Tst>>::type;
+                    // groups of 4 samples; those before position 0, which starts a group, read as zeros
+                    constexpr int V = 4, NV = S::DOUT / V;
+                    using Raw = rawv_st<Tst, 4>;
                     auto load_bin = [&](Raw (&r)[NV], int pos) {
 #pragma unroll
-                        for (int i = 0; i < NV; i++) {
-                            const Tst *q = row + max(pos + V * i, 0);
-                            if constexpr (V == 4)
-                                r[i] = ldv_raw<Tst, 4>(q);
-                            else
-                                r[i] = ld_raw(q);
-                        }
+                        for (int i = 0; i < NV; i++)
+                            r[i] = ldv_raw<Tst, 4>(row + max(pos + V * i, 0));
                     };
                     auto floats = [&](const Raw (&r)[NV], int pos, float (&y)[S::DOUT]) {
 #pragma unroll
                         for (int i = 0; i < NV; i++) {
-                            if constexpr (V == 4)
-                                from_rawv<Tst, 4>(r[i], y + 4 * i);
-                            else
-                                y[i] = from_raw<Tst>(r[i]);
+                            from_rawv<Tst, 4>(r[i], y + 4 * i);
 #pragma unroll
                             for (int q = 0; q < V; q++)
                                 y[V * i + q] = (pos + V * i >= 0) ? y[V * i + q] : 0.0f;
@@ -768,6 +765,9 @@ k_pf(PfArgs a)
     }
 }
 
+// Output bins that the two-step kernel is built for (see pf_two_step).
+static constexpr bool pf_has_two_step(int dout) { return dout == 8 || dout == 16; }
+
 template<typename Tst, int LW>
 static void launch_pf_lw(const PfArgs &a, hipStream_t st, dim3 grid)
 {
@@ -776,9 +776,14 @@ static void launch_pf_lw(const PfArgs &a, hipStream_t st, dim3 grid)
 #define PDD_PF(LDV)                                                                \
         case (1 << LDV):                                                           \
             if (a.out_var)                                                         \
-                hipLaunchKernelGGL((k_pf_var<Tst, LW, LDV>), grid, block, 0, st, a);  \
-            else                                                                   \
-                hipLaunchKernelGGL((k_pf<Tst, LW, LDV>), grid, block, 0, st, a); \
+                hipLaunchKernelGGL((k_pf_one<Tst, LW, LDV, true>), grid, block, 0, st, a);  \
+            else if constexpr (pf_has_two_step(1 << LDV)) {                                      \
+                if (a.two_step)                                                    \
+                    hipLaunchKernelGGL((k_pf<Tst, LW, LDV>), grid, block, 0, st, a); \
+                else                                                               \
+                    hipLaunchKernelGGL((k_pf_one<Tst, LW, LDV, false>), grid, block, 0, st, a); \
+            } else                                                                 \
+                hipLaunchKernelGGL((k_pf_one<Tst, LW, LDV, false>), grid, block, 0, st, a); \
             break;
         PDD_PF(0) PDD_PF(1) PDD_PF(2) PDD_PF(3) PDD_PF(4) PDD_PF(5)
 #undef PDD_PF
@@ -786,22 +791,55 @@ static void launch_pf_lw(const PfArgs &a, hipStream_t st, dim3 grid)
     }
 }
 
-// Time segments per chunk: the fewest (a power of two) that give at least a.target_blocks
-// workgroups (2048 unless tuned), within segments of whole tiles of at least
-// nwarm*TL positions (see rotate_rows). With out_var, one segment.
-static int pf_nseg(const PfArgs &a, long nblocks, int TL)
+// Two steps or one. Step 2 walks NBACK + 1 bins per output bin, spread over the M multiplets of a DM
+// row, so it pays with many multiplets and long bins. Medians of kernel times, one step and two, us:
+//   (NBACK + 1) / M   one    two    (2048 samples, float32 and float16)
+//   0.12, M 16        112    81     109    68       boxcars up to 4, bins of 16
+//   0.31, M 16        130    104    125    94       16, bins of 8
+//   0.62, M 8         126    109    122    102      16, bins of 8
+//   1.12, M 8         135    150    127    128      32, bins of 8
+//   2.25, M 4         84     97     75     82       16, bins of 4
+//   4.25, M 4         97     186    85     125      32, bins of 4
+// Bins of 4 went from 27% slower to 20% faster and seldom occur with 16 multiplets or more; bins of 1
+// and 2 were up to 3.2 times slower, and with bins of 32 the unrolled walks spill (up to 7 times slower).
+// Small launches are bounded by latency: the tiles of one step are shorter, those of two steps pass
+// without a barrier, which counts more the longer the warm-up is. Up to 2^14 positions of a
+// workgroup's chunk and boxcars of 2 to 8 samples, one step took 9 to 16 us and two steps 13 to 19;
+// with boxcars of 16 and 32 16 and 29 against 14 and 27 (float16 17 and 23).
+static bool pf_two_step(const PfArgs &a, long nblocks, int TL)
+{
+    if (a.out_var || !pf_has_two_step(a.Dout) || a.Tp % TL != 0 || a.two_step == 0)
+        return false;
+    if (a.two_step > 0)
+        return true;
+    const int wmax = 1 << ((a.P - 1) / 3);
+    const int bins = (a.tpad + a.Dout - 1) / a.Dout + 1;       // NBACK + 1
+    return 10 * bins <= 7 * a.M && (wmax >= 16 || nblocks * a.Tp > (1 << 14));
+}
+
+// Time segments per chunk, of whole tiles and at least nwarm of them (see rotate_rows). One step: the
+// fewest that give at least a.target_blocks workgroups (2048 unless tuned). Two steps: up to that number, the one
+// with the shortest rounds of resident workgroups (three per CU) times tiles walked, warm-up
+// among them: with 32 workgroups of 1024 float32 samples 16 segments take 24 us, 32 segments (64 positions walked
+// for 32) 33 us; 512 workgroups of 2048 samples, 3 segments 279 us, 6 segments 277, 8 288 us. With out_var, one segment.
+static int pf_nseg(const PfArgs &a, bool two_step, long nblocks, int TL)
 {
     if (a.out_var)
         return 1;
-    const int nwarm = (a.tpad + TL - 1) / TL;
-    int nseg = 1;
-    while (nblocks * nseg < a.target_blocks) {
-        const int n2 = 2 * nseg;
-        if (a.Tp % (TL * n2) != 0 || a.Tp / n2 < nwarm * TL)
-            break;
-        nseg = n2;
+    const int ntiles = a.Tp / TL, nwarm = (a.tpad + TL - 1) / TL;
+    const int most = int(std::min<long>(std::max(1, ntiles / nwarm), (a.target_blocks + nblocks - 1) / nblocks));
+    if (!two_step)
+        return most;
+    int best = 1;
+    long cost = 0;
+    for (int n = 1; n <= most; n++) {
+        const long c = ((nblocks * n + 767) / 768) * ((ntiles + n - 1) / n + nwarm);
+        if (n == 1 || c < cost) {
+            best = n;
+            cost = c;
+        }
     }
-    return nseg;
+    return best;
 }
 
 template<typename Tst>
@@ -810,7 +848,9 @@ static void launch_pf_t(const PfArgs &a0, hipStream_t st)
     PfArgs a = a0;
     const int ndpf = kPfThreads / a.M;
     const unsigned nbx = unsigned((a.ndm_out + ndpf - 1) / ndpf);
-    a.nseg = pf_nseg(a, long(nbx) * a.B, kPfLine / int(sizeof(Tst)));
+    constexpr int TL2 = kPfLine / int(sizeof(Tst));      // k_pf's tile
+    a.two_step = pf_two_step(a, long(nbx) * a.B, TL2);
+    a.nseg = pf_nseg(a, a.two_step, long(nbx) * a.B, a.two_step ? TL2 : pf_tile_len(a.Dout));
     dim3 grid{nbx, unsigned(a.B), unsigned(a.nseg)};
     switch ((a.P - 1) / 3) {
         case 0: launch_pf_lw<Tst, 0>(a, st, grid); break;

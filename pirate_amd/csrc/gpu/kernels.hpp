@@ -115,7 +115,8 @@ struct PfArgs {
     int B, ndm_out, M, N, P, nlev, Tp, Dout, Dcore, ndm_wt, nt_wt, nt_out;
     int beam0;                // global index of the batch's first beam (sb rows are per global beam)
     int nseg = 1;             // time segments per chunk (set by launch_pf)
-    long target_blocks = 2048;   // launch_pf picks the fewest segments giving this many workgroups
+    int two_step = -1;        // two-step kernel: -1 by launch_pf's rule, 0 never, 1 wherever there is one
+    long target_blocks = 2048;   // launch_pf picks at most the fewest segments giving this many workgroups
     double *out_var = nullptr;   // optional (B, ndm_out, M, P) float64: per-chunk mean square of each
                                  // (multiplet, profile)'s weighted candidates
 };

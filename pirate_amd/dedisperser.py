@@ -347,7 +347,7 @@ class GpuDedisperser:
 
     def set_tuning(self, name, value):
         """Sets a launch shape that changes no output, only speed: 'pf_target_blocks',
-        'grid_xcd_run' or 'fork' (see include/pirate_amd.h); applies from the next launch."""
+        'pf_two_step', 'grid_xcd_run' or 'fork' (see include/pirate_amd.h); applies from the next launch."""
         L.check(L.lib().pdd_dedisperser_set_tuning(self._h, name.encode(), int(value)))
 
     def apply_tuning_table(self, table=None):

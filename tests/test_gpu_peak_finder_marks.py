@@ -1,6 +1,7 @@
-"""The two-step peak finder where values leave the range in which its first step is exact, bit for
-bit against the kernel that visits every candidate in order (the one that also forms the float64
-variances): boxcar sums of finite samples that overflow, with zero weights on some profiles."""
+"""The peak finder in one and in two steps, and by the rule between them, bit for bit against the
+kernel that also forms the float64 variances, which visits every candidate in order in one time
+segment: where values leave the range in which the two-step kernel's first step is exact, and
+over bin lengths, boxcar lengths, multiplets and chunks that the time segments do not divide."""
 
 import numpy as np
 import pytest
@@ -11,18 +12,21 @@ from gpu_harness import random_weights
 pytestmark = pytest.mark.gpu
 
 
-def make_pair(rank, bands, widths, dtype, B, T, time_ds=0):
-    """The same search with the peak finder proper and with the one that forms variances."""
+def make_all(rank, bands, widths, dtype, B, T, time_ds=0):
+    """The same search with the two-step kernel (where there is one), with one step, by the rule
+    between the two, and with the one that forms variances."""
     import pirate_amd as pa
-    trees = [dict(pt(0, w, min(64, 2**(rank - 1)), 64), time_downsampling=time_ds) for w in widths]
+    trees = [dict(pt(0, w, min(64, 2**(rank - 1)), min(64, (T >> p) & -(T >> p))), time_downsampling=time_ds)
+             for p, w in enumerate(widths)]
     cfg = dict(BASE, dtype=dtype, zone_nfreq=[2**rank], zone_freq_edges=[400, 800], toplevel_tree_rank=rank,
                time_samples_per_chunk=T, beams_per_gpu=B, beams_per_batch=B, num_active_batches=1,
                frequency_subband_counts=bands, primary_trees=trees)
     plan = pa.DedispersionPlan(pa.DedispersionConfig.from_dict(cfg))
-    dds = [pa.GpuDedisperser(plan, enable_variances=v) for v in (False, True)]
+    dds = [pa.GpuDedisperser(plan, enable_variances=v) for v in (False, False, False, True)]
     rng = np.random.default_rng(rank)
-    for dd in dds:
+    for dd, two_step in zip(dds, (1, 0, -1, -1)):
         dd.allocate()
+        dd.set_tuning('pf_two_step', two_step)
     for it in range(plan.ntrees):
         w = random_weights(rng, dds[0], it)
         for dd in dds:
@@ -31,7 +35,7 @@ def make_pair(rank, bands, widths, dtype, B, T, time_ds=0):
 
 
 def outputs(plan, dds, c, x):
-    """Bit patterns of (out_max, out_argmax) of every tree, for each of the two."""
+    """Bit patterns of (out_max, out_argmax) and values of every tree, for each of the dedispersers."""
     import torch
     x = torch.from_numpy(x).cuda()
     bits = torch.int32 if plan.dtype == 'float32' else torch.int16
@@ -48,8 +52,9 @@ def outputs(plan, dds, c, x):
 def assert_equal(plan, res, c):
     for it in range(plan.ntrees):
         for i, what in enumerate(('out_max', 'out_argmax')):
-            a, b = res[0][it][i], res[1][it][i]
-            assert np.array_equal(a, b), f'chunk {c} tree {it} {what}: {int(np.sum(a != b))} of {a.size} differ'
+            b = res[-1][it][i]
+            for a, name in zip((r[it][i] for r in res[:-1]), ('two steps', 'one step', 'rule')):
+                assert np.array_equal(a, b), f'{name}: chunk {c} tree {it} {what}: {int(np.sum(a != b))} of {a.size} differ'
 
 
 # bins of 16, 8 and 16 samples; 16, 34 and 91 multiplets
@@ -63,7 +68,7 @@ def test_sums_that_overflow(rank, bands, dtype):
     third profile of one level."""
     B, T = 2, 512
     print(f'[peak finder marks] overflow rank {rank} {bands} {dtype}', flush=True)
-    plan, dds = make_pair(rank, bands, [16], dtype, B, T)
+    plan, dds = make_all(rank, bands, [16], dtype, B, T)
     bin_len = T // plan.trees[0].nt_out
     rng = np.random.default_rng(1)
     w = np.zeros(dds[0].wt_shape(0), dtype=np.float32)          # (slots, B, ndm_wt, nt_wt, P, N)
@@ -80,4 +85,22 @@ def test_sums_that_overflow(rank, bands, dtype):
                 v[b, :, k * bin_len - 1:k * bin_len + 1] = -1.72e38
         x = (v * 2.0 ** (-rank / 2)).astype(np.float32)
         res = outputs(plan, dds, c, x)
+        assert_equal(plan, res, c)
+
+
+# (rank, subband counts, boxcars, chunk, beams): 1 to 63 tiles per chunk, launches on both sides of the rule
+SEGMENTS = [
+    (4, [1], [32], 1984, 3), (8, [1], [16, 4], 1408, 1), (8, [2, 2, 1], [32], 4032, 2), (10, [1], [2], 320, 4),
+    (10, [3, 3, 1], [16, 8], 1408, 1), (12, [1], [32, 1], 2944, 1), (14, [1], [16], 64, 1), (14, [1], [8], 1984, 1),
+]
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'float16'])
+@pytest.mark.parametrize('rank,bands,widths,T,B', SEGMENTS)
+def test_segments(rank, bands, widths, T, B, dtype):
+    print(f'[peak finder marks] segments rank {rank} {bands} {widths} T {T} B {B} {dtype}', flush=True)
+    plan, dds = make_all(rank, bands, widths, dtype, B, T)
+    rng = np.random.default_rng(2)
+    for c in range(3):
+        res = outputs(plan, dds, c, rng.standard_normal((B, plan.nfreq, T)).astype(np.float32))
         assert_equal(plan, res, c)
