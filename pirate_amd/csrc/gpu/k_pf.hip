@@ -511,7 +511,11 @@ k_pf_one(PfArgs a)
 // stream over the bin again with PfLane, which gives the value and the token of the first
 // maximum. A DM row has M streams, so step 2 costs 1/M of a full walk per stream.
 // Infinities, NaN and samples that could make a sum overflow (pf_wild): a stream is marked in each
-// bin whose windows hold one, and step 2 walks every stream of a marked (DM row, bin) with PfLane.
+// bin whose windows hold one. A wave with a marked lane walks that bin with PfLane in place of
+// PfMax, from the same windows, and leaves value and token for step 2, which then walks nothing
+// for a winner that has its token. So data full of NaN costs about what the walk of every candidate
+// costs; with all M streams of a marked (DM row, bin) walked by one lane of step 2 it cost up to 4.7
+// times that.
 //
 // Samples reach LDS by direct loads (no registers, no conversion), 128 bytes of a row at a
 // time, so that every line is fetched once; a wave stages the 64 rows that its lanes walk, so
@@ -519,7 +523,7 @@ k_pf_one(PfArgs a)
 // this one. One load instruction brings 8 rows x 128 bytes; lane i of the
 // instruction writes the i-th 16 bytes, so the 16-byte chunks of a row are permuted on the
 // global side (slot s of row r holds chunk s ^ (r & 7)), and the 16-byte reads of 8
-// neighbouring rows cover all banks. 49 KB of LDS and 168 VGPRs: three workgroups (12 waves)
+// neighbouring rows cover all banks. 51 KB of LDS and 168 VGPRs: three workgroups (12 waves)
 // per CU. Bounded by VALU issue (about 400 instructions per stream and 16-sample bin at Wmax 16,
 // against 520 with every candidate compared) and, for float32, near half by the row reads.
 // 16384 DM rows x 2048 samples x 16 beams, Wmax 16, bins of 16: float32 0.774 -> 0.547 ms,
@@ -547,7 +551,7 @@ k_pf(PfArgs a)
     static_assert(TL % SB == 0 && BPS <= kPfBatch, "whole bins per tile");
     __shared__ __align__(16) unsigned char tile[kPfThreads * kPfLine];
     __shared__ float rv[kPfBatch * RVS];
-    __shared__ unsigned char rl[kPfBatch * RLS];
+    __shared__ unsigned short rc[kPfBatch * RLS];     // code: 0x8000 if walked with PfLane | level << 12 | its token
     __shared__ int sn[kPfThreads];               // weight column of each stream
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -634,20 +638,40 @@ k_pf(PfArgs a)
             if (active) {
 #pragma unroll
                 for (int j = 0; j < BPS; j++) {
-                    // loaded here, used at the end of the bin; kept from bin to bin they would
-                    // be live across step 2, which spills
-                    float wt[S::P];
                     const float *wp = wrow + long((tbs + j) / Tds) * S::P * N;
-#pragma unroll
-                    for (int p = 0; p < S::P; p++)
-                        wt[p] = wp[p * N];
                     marked = pf_wild<S::DOUT>(x + j * S::DOUT) ? NBACK + 1 : max(marked - 1, 0);
-                    ln.template bin<true>(x + j * S::DOUT);
                     float V;
-                    unsigned int lev;
-                    ln.combine(wt, V, lev);
+                    unsigned int code;
+                    // (expected: as equals, the two walks are given registers that spill at Wmax 8 and 32)
+                    if (__builtin_expect(!__any(marked > 0), 1)) {
+                        // loaded here, used at the end of the bin; kept from bin to bin they would
+                        // be live across step 2, which spills
+                        float wt[S::P];
+#pragma unroll
+                        for (int p = 0; p < S::P; p++)
+                            wt[p] = wp[p * N];
+                        ln.template bin<true>(x + j * S::DOUT);
+                        unsigned int lev;
+                        ln.combine(wt, V, lev);
+                        code = lev << 12;
+                    } else {
+                        PfLane<S, false> le;
+#pragma unroll
+                        for (int i = 0; i < S::WTOT; i++)
+                            le.w[i] = ln.w[i];
+#pragma unroll
+                        for (int p = 0; p < S::P; p++)
+                            le.wt[p] = wp[p * N];
+                        le.template bin<true>(x + j * S::DOUT);
+#pragma unroll
+                        for (int i = 0; i < S::WTOT; i++)
+                            ln.w[i] = le.w[i];
+                        unsigned int c;
+                        le.combine(V, c);
+                        code = 0x8000u | (unsigned(pf_level_of_token(c)) << 12) | c;
+                    }
                     rv[(nbatch + j) * RVS + tid] = V;
-                    rl[(nbatch + j) * RLS + tid] = (unsigned char)((marked > 0) ? 0x80u : lev);
+                    rc[(nbatch + j) * RLS + tid] = (unsigned short)(code);
                 }
             }
             nbatch += BPS;
@@ -662,56 +686,51 @@ k_pf(PfArgs a)
             for (int idx = wave_local ? lane : tid; idx < nd2 * nbatch; idx += wave_local ? 64 : kPfThreads) {
                 const int d = idx / nbatch + d2, j = idx % nbatch;
                 const float *pv = rv + j * RVS + d * M;
-                const unsigned char *pl = rl + j * RLS + d * M;
+                const unsigned short *pc = rc + j * RLS + d * M;
                 float V = pv[0];
-                int key = pl[0] * M, m0 = 0;
-                bool all = (pl[0] & 0x80) != 0;
+                unsigned int code = pc[0];
+                int key = int((code >> 12) & 7) * M, m0 = 0;
 #pragma unroll 4
                 for (int mm = 1; mm < M; mm++) {
                     const float v = pv[mm];
-                    const int lv = pl[mm], k = lv * M + mm;
-                    all |= (lv & 0x80) != 0;
+                    const unsigned int c = pc[mm];
+                    const int k = int((c >> 12) & 7) * M + mm;
                     if (v > V || (v == V && k < key)) {
                         V = v;
                         key = k;
+                        code = c;
                         m0 = mm;
                     }
                 }
-                const int m1 = all ? M : m0 + 1;
-                m0 = all ? 0 : m0;
 
                 const int tb = tbb + j;
-                const float *wp = wbeam + (long((dpf0 + d) / Wds) * a.nt_wt + tb / Tds) * S::P * N;
-                float bv = 0.0f;
-                unsigned int bt = 0;
-                int bk = 0;
-#pragma unroll 1
-                for (int mm = m0; mm < m1; mm++) {
+                unsigned int tok = code & 0xfffu;
+                if (!(code & 0x8000u)) {
+                    const float *wq = wbeam + (long((dpf0 + d) / Wds) * a.nt_wt + tb / Tds) * S::P * N + sn[d * M + m0];
                     PfLane<S, false> pl2;
 #pragma unroll
                     for (int i = 0; i < S::WTOT; i++)
                         pl2.w[i] = 0.0f;
-                    const float *wq = wp + sn[d * M + mm];
 #pragma unroll
                     for (int p = 0; p < S::P; p++)
                         pl2.wt[p] = wq[p * N];
-                    const Tst *row = rows + long(d * M + mm) * a.rowlen;
+                    const Tst *row = rows + long(d * M + m0) * a.rowlen;
                     const int pb = a.tpad + tb * S::DOUT;
                     // groups of 4 samples; those before position 0, which starts a group, read as zeros
-                    constexpr int V = 4, NV = S::DOUT / V;
+                    constexpr int VL = 4, NV = S::DOUT / VL;
                     using Raw = rawv_st<Tst, 4>;
                     auto load_bin = [&](Raw (&r)[NV], int pos) {
 #pragma unroll
                         for (int i = 0; i < NV; i++)
-                            r[i] = ldv_raw<Tst, 4>(row + max(pos + V * i, 0));
+                            r[i] = ldv_raw<Tst, 4>(row + max(pos + VL * i, 0));
                     };
                     auto floats = [&](const Raw (&r)[NV], int pos, float (&y)[S::DOUT]) {
 #pragma unroll
                         for (int i = 0; i < NV; i++) {
                             from_rawv<Tst, 4>(r[i], y + 4 * i);
 #pragma unroll
-                            for (int q = 0; q < V; q++)
-                                y[V * i + q] = (pos + V * i >= 0) ? y[V * i + q] : 0.0f;
+                            for (int q = 0; q < VL; q++)
+                                y[VL * i + q] = (pos + VL * i >= 0) ? y[VL * i + q] : 0.0f;
                         }
                     };
                     float y[S::DOUT];
@@ -739,23 +758,15 @@ k_pf(PfArgs a)
                         floats(r, pb, y);
                     }
                     pl2.template bin<true>(y);
-                    float v;
-                    unsigned int c;
-                    pl2.combine(v, c);
-                    const int k = pf_level_of_token(c) * M + mm;
-                    if (mm == m0 || v > bv || (v == bv && k < bk)) {
-                        bv = v;
-                        bt = c | (unsigned(mm) << 16);
-                        bk = k;
-                    }
+                    pl2.combine(V, tok);
                 }
                 const long o = long(dpf0 + d) * a.nt_out + tb;
-                st_st(outm + o, bv);
-                outa[o] = bt;
+                st_st(outm + o, V);
+                outa[o] = tok | (unsigned(m0) << 16);
             }
             nbatch = 0;
             if (!wave_local)
-                __syncthreads();       // rv and rl are free
+                __syncthreads();       // rv and rc are free
         }
     }
 

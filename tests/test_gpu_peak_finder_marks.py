@@ -104,3 +104,46 @@ def test_segments(rank, bands, widths, T, B, dtype):
     for c in range(3):
         res = outputs(plan, dds, c, rng.standard_normal((B, plan.nfreq, T)).astype(np.float32))
         assert_equal(plan, res, c)
+
+
+# (rank, subband counts, boxcars, output bin or 0): 2 to 91 multiplets, bins of 1 to 32 samples
+SHAPES = {
+    'm4_bins1': (8, [1], [32], 1), 'm2_bins2': (4, [1], [16], 2), 'm10_bins4': (8, [2, 2, 1], [16, 4], 0),
+    'm8_bins8': (10, [1], [32, 2], 0), 'm34_bins8': (11, [4, 5, 3, 1], [8, 32], 0), 'm16_bins16': (13, [0, 0, 0, 0, 1], [16, 8], 0),
+    'm91_bins16': (14, [5, 9, 7, 3, 1], [16], 0), 'm8_bins32': (10, [1], [16], 32),
+}
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'float16', 'bfloat16'])
+@pytest.mark.parametrize('name', list(SHAPES))
+def test_sparse_marks(name, dtype):
+    """Three infinities or NaN per beam and chunk, so that marked and clean bins and streams lie side by
+    side, on inputs of few values (1 or 2 in one of 50 dedispersed samples), all weights 1: the
+    largest value occurs in several multiplets and profiles."""
+    rank, bands, widths, time_ds = SHAPES[name]
+    B, T = 2, 512
+    print(f'[peak finder marks] sparse {name} {dtype}', flush=True)
+    plan, dds = make_all(rank, bands, widths, dtype, B, T, time_ds)
+    for it in range(plan.ntrees):
+        for dd in dds:
+            dd.fill_all_weights(it, np.ones(dd.wt_shape(it), dtype=np.float32))
+    rng = np.random.default_rng(4)
+    finite, bad, tied = (np.zeros(plan.ntrees, dtype=int) for _ in range(3))
+    for c in range(4):
+        x = np.zeros((B, plan.nfreq, T), dtype=np.float32)
+        n = max(1, int(0.02 * x.size / plan.nfreq))
+        x.reshape(-1)[rng.choice(x.size, n, replace=False)] = rng.integers(1, 3, size=n)
+        if c > 0:
+            for b in range(B):
+                # one at each end of the band: at one of them no DM delays it past the last chunk
+                for f, v in zip((0, plan.nfreq - 1, rng.integers(plan.nfreq)), rng.choice([np.inf, -np.inf, np.nan], 3)):
+                    x[b, f, rng.integers(T)] = v
+        res = outputs(plan, dds, c, x)
+        assert_equal(plan, res, c)
+        for it in range(plan.ntrees):
+            v = res[0][it][2]
+            finite[it] += np.sum(np.isfinite(v))
+            bad[it] += np.sum(~np.isfinite(v))
+            # the same nonzero maximum in neighbouring DM rows: multiplets of both share its samples
+            tied[it] += np.sum((v[:, 1:] == v[:, :-1]) & (v[:, 1:] > 0))
+    assert np.all(finite > 0) and np.all(bad > 0) and np.all(tied > 0), (finite, bad, tied)
