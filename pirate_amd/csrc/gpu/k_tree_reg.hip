@@ -92,7 +92,7 @@ struct RegDims {
     static constexpr int WLA = (OVA + U) / S, WL = (OV + U) / 2;         // lanes of a window
     static constexpr int T2 = NRB * (NRB - 1) / 2;
     static constexpr int SUMB = NRA * (NRA - 1) / 2;         // sum of bitrev(j) over j
-    static constexpr int NRES = T2 * SUMB + D * OV;           // saved line samples
+    static constexpr int NRES = (T2 * SUMB + D * OV + 1) & ~1;     // saved line samples (an odd number at rank 2)
     // and the histories, or the last input samples (stage 1)
     static constexpr int NSTATE = NRES + (HIST ? NRB * Sub<K1>::NST : D * OVA);
     static constexpr int LMAX = (NRB - 1) * (NRA - 1);
@@ -101,6 +101,7 @@ struct RegDims {
     static constexpr int WARM = (LMAX + OV + (HIST ? NRA - 1 : 0) + U - 1) / U;
     static_assert(WLA <= 64 && WL <= 64, "a window fits a wave");
     static_assert(OVA <= kTreeOverlap, "ring capacities");
+    static_assert(HIST || (NRES % 2 == 0 && NSTATE % 2 == 0), "saved input samples are read and written in aligned pairs");
 
     // Line (h, j): even(lag) + OV + U floats, j-major, so that every line starts 8-byte aligned.
     static constexpr int LINE0 = OV + U;
