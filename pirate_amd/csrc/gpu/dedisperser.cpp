@@ -274,6 +274,7 @@ void GpuDedisperser::allocate()
     host_ring.assign(npri, nullptr);
     s1_state.resize(npri);
     s1_state_bstride.resize(npri);
+    s1_nseg.resize(npri);
     const long max_gpu_clag = plan->config.max_gpu_clag;
     for (long p = 0; p < npri; p++) {
         const int dd1 = int(plan->stage1_dd_rank[p]), amb1 = int(plan->stage1_amb_rank[p]);
@@ -283,7 +284,7 @@ void GpuDedisperser::allocate()
         long tot = 0;
         for (long a1 = 0; a1 < pow2(amb1); a1++)
             for (long j = 0; j < pow2(dd1); j++) {
-                long maxlag = 0, minlag = -1;
+                long maxlag = 0, minlag = -1, overlap = 0;
                 for (long it = 0; it < ntrees; it++) {
                     const DedispersionTree &t = plan->trees[it];
                     if (t.primary_tree_index != p || a1 >= pow2(t.dd_rank))
@@ -291,12 +292,13 @@ void GpuDedisperser::allocate()
                     const long lag = rb_lag(a1, j, t.amb_rank, t.dd_rank, p > 0);
                     maxlag = std::max(maxlag, lag);
                     minlag = (minlag < 0) ? lag : std::min(minlag, lag);
+                    overlap = std::max(overlap, long(tree_overlap(t.dd_rank)));
                 }
                 long r = a1 * pow2(dd1) + j;
                 if (minlag >= 0 && max_gpu_clag < (1L << 40))
                     kr[r] = std::max(0L, minlag / Tp - max_gpu_clag);
                 // rows of whole 128-byte lines (16-bit rows of 64 bytes: stages 1 and 2 1 to 2% slower)
-                cap[r] = align_up(maxlag - kr[r] * Tp + Tp + kTreeOverlap, 128 / elt_bytes);
+                cap[r] = align_up(maxlag - kr[r] * Tp + Tp + overlap, 128 / elt_bytes);
                 off[r] = tot;
                 tot += cap[r];
             }
@@ -328,8 +330,8 @@ void GpuDedisperser::allocate()
         host_bstride[p] = align_up(hoff, 64);
         spill_k[p] = kr;
         ring_bstride[p] = align_up(inbox_off[p] + nspill[p] * Tp, 64);
-        PDD_CHECK(ring_bstride[p] < (1L << 31), "GpuDedisperser: lag ring of primary tree " << p
-                  << " exceeds 2^31 elements per beam (tree kernels use 32-bit row offsets)");
+        PDD_CHECK(ring_bstride[p] < (1L << 32), "GpuDedisperser: lag ring of primary tree " << p
+                  << " exceeds 2^32 elements per beam (tree kernels use 32-bit row offsets)");
         rings[p] = dalloc(size_t(total_beams) * ring_bstride[p] * elt_bytes);
         ring_row_off[p] = up_long(off);
         ring_row_cap[p] = up_long(cap);
@@ -342,7 +344,8 @@ void GpuDedisperser::allocate()
             std::memset(host_ring[p], 0, hb);
             host_bytes_allocated += hb;
         }
-        s1_state_bstride[p] = 2 * pow2(amb1) * tree_state_nelts(int(dd1));      // two chunk parities
+        s1_nseg[p] = tree_segments(dd1, pow2(amb1) * B, int(Tp));
+        s1_state_bstride[p] = pow2(amb1) * tree_state_nelts(dd1, false, s1_nseg[p]);
         s1_state[p] = dalloc(size_t(total_beams) * s1_state_bstride[p] * sizeof(float));
     }
 
@@ -351,6 +354,7 @@ void GpuDedisperser::allocate()
     d_m_to_n.resize(ntrees);
     s2_state.resize(ntrees);
     s2_state_bstride.resize(ntrees);
+    s2_nseg.resize(ntrees);
     weights.resize(ntrees);
     out_max.resize(ntrees);
     out_argmax.resize(ntrees);
@@ -371,7 +375,8 @@ void GpuDedisperser::allocate()
                   << " exceed 2^31 elements per beam");
         sb[it] = dalloc((size_t(total_beams) * t.ndm_out * T.M * T.rowlen + T.lead) * elt_bytes);
         d_m_to_n[it] = up_int(T.m_to_n);
-        s2_state_bstride[it] = 2 * pow2(t.amb_rank) * tree_state_nelts(t.dd_rank);      // two chunk parities
+        s2_nseg[it] = tree_segments(t.dd_rank, pow2(t.amb_rank) * B, int(t.nt_ds));
+        s2_state_bstride[it] = pow2(t.amb_rank) * tree_state_nelts(t.dd_rank, true, s2_nseg[it]);
         s2_state[it] = dalloc(size_t(total_beams) * s2_state_bstride[it] * sizeof(float));
         weights[it] = dalloc(size_t(nbatches_wt) * B * t.ndm_wt * t.nt_wt * t.nprofiles * T.N * sizeof(float));
         // out_max / out_argmax: views into the output region (below)
@@ -576,6 +581,7 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
         s.ring.bstride = ring_bstride[p];
         s.state = (float *) s1_state[p].ptr;
         s.state_bstride = s1_state_bstride[p];
+        s.nseg = s1_nseg[p];
         s.B = int(B);
         s.amb = int(plan->stage1_amb_rank[p]);
         s.dd = int(plan->stage1_dd_rank[p]);
@@ -616,6 +622,7 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
             }
             s2.state = (float *) s2_state[it].ptr;
             s2.state_bstride = s2_state_bstride[it];
+            s2.nseg = s2_nseg[it];
             s2.B = int(B);
             s2.amb = t.amb_rank;
             s2.dd = t.dd_rank;

@@ -210,8 +210,8 @@ private:
     std::vector<DeviceArray> sb;      // [itree] (B, ndm_out, M, rowlen)
     std::vector<DeviceArray> d_m_to_n;
     DeviceArray lds_state;  long lds_state_bstride = 0;
-    std::vector<DeviceArray> s1_state; std::vector<long> s1_state_bstride;
-    std::vector<DeviceArray> s2_state; std::vector<long> s2_state_bstride;
+    std::vector<DeviceArray> s1_state; std::vector<long> s1_state_bstride; std::vector<int> s1_nseg;
+    std::vector<DeviceArray> s2_state; std::vector<long> s2_state_bstride; std::vector<int> s2_nseg;
     std::vector<DeviceArray> weights; // [itree] (nbatches_wt, B, ndm_wt, nt_wt, P, N) float
     std::vector<DeviceArray> out_max, out_argmax;   // [itree] (nbatches_out, B, ndm_out, nt_out), views into out_region
     DeviceArray out_region;

@@ -93,15 +93,14 @@ struct RegDims {
     static constexpr int T2 = NRB * (NRB - 1) / 2;
     static constexpr int SUMB = NRA * (NRA - 1) / 2;         // sum of bitrev(j) over j
     static constexpr int NRES = (T2 * SUMB + D * OV + 1) & ~1;     // saved line samples (an odd number at rank 2)
-    // and the histories, or the last input samples (stage 1)
-    static constexpr int NSTATE = NRES + (HIST ? NRB * Sub<K1>::NST : D * OVA);
+    // and the histories, or stage 1's last input samples
+    static constexpr int nstate(bool stage2) { return NRES + (HIST ? NRB * Sub<K1>::NST : stage2 ? 0 : D * OVA); }
     static constexpr int LMAX = (NRB - 1) * (NRA - 1);
     // tiles that fill a segment's lines (lag + OV samples), with histories from outputs that no
     // longer depend on the zeros it started with (the first NRA - 1 samples do)
     static constexpr int WARM = (LMAX + OV + (HIST ? NRA - 1 : 0) + U - 1) / U;
     static_assert(WLA <= 64 && WL <= 64, "a window fits a wave");
-    static_assert(OVA <= kTreeOverlap, "ring capacities");
-    static_assert(HIST || (NRES % 2 == 0 && NSTATE % 2 == 0), "saved input samples are read and written in aligned pairs");
+    static_assert(HIST || (NRES % 2 == 0 && nstate(false) % 2 == 0), "saved input samples are read and written in aligned pairs");
 
     // Line (h, j): even(lag) + OV + U floats, j-major, so that every line starts 8-byte aligned.
     static constexpr int LINE0 = OV + U;
@@ -247,6 +246,9 @@ struct RawTwo16 {
 template<> struct RawS<__half, 2> : RawTwo16<__half> { };
 template<> struct RawS<__hip_bfloat16, 2> : RawTwo16<__hip_bfloat16> { };
 
+// Element offset of a ring row held by lane k: up to 2^32 elements per beam.
+__device__ __forceinline__ unsigned lane_offset(int v, int k) { return unsigned(__builtin_amdgcn_readlane(v, k)); }
+
 __device__ __forceinline__ int rowlen_of(const Stage1Args &) { return 0; }
 __device__ __forceinline__ int rowlen_of(const Stage2Args &a) { return a.rowlen; }
 __device__ __forceinline__ int nband_of(const Stage1Args &, int) { return 0; }
@@ -272,9 +274,10 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
     const int first = int(blockIdx.z) * ntiles / a.nseg, end = (int(blockIdx.z) + 1) * ntiles / a.nseg;
     const int start = blockIdx.z ? first - F::WARM : 0;       // >= 0: the host checks it
 
-    // state, double-buffered by chunk parity (segment 0 reads what the last segment writes)
-    const long half_state = a.state_bstride >> 1;
-    float *st = a.state + gbeam * a.state_bstride + long(tr) * F::NSTATE;
+    // state: one segment reads and writes it in place, several keep it twice by chunk parity (segment
+    // 0 reads what the last one writes)
+    const long half_state = (a.nseg > 1) ? a.state_bstride >> 1 : 0;
+    float *st = a.state + gbeam * a.state_bstride + long(tr) * F::nstate(STAGE2);
     const float *rd = st + (chunk & 1) * half_state;
     float *wr = st + ((chunk + 1) & 1) * half_state;
 
@@ -316,7 +319,8 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
     // position of the next tile; stage 2 reads the rows of its phase-A sub-trees (lane s*NRA + l) at
     // their lag, from the start of the next tile's window. A tile that no row wraps in takes one
     // lane read per row and scalar addresses.
-    int roff, rpos, rcap;
+    unsigned roff;
+    int rpos, rcap;
     {
         long rr, t = chunk * a.Tp + start * U;
         if constexpr (!STAGE2) {
@@ -327,7 +331,7 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
             t -= a.row_lag[rr] + F::OVA;
         }
         const long cap = a.ring.row_cap[rr];
-        roff = int(a.ring.row_off[rr]);
+        roff = unsigned(a.ring.row_off[rr]);
         rpos = int(ring_pos(t, cap));
         rcap = int(cap);
     }
@@ -366,10 +370,10 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
             }
         } else {
             const unsigned tb = unsigned(i) * unsigned(sizeof(Tst));
-            const int q = roff + rpos;
+            const int q = int(roff + unsigned(rpos));
             const unsigned long long wrap = __ballot(rpos + wlen > rcap);
             auto load_row = [&](int s, int l) {
-                const Tst *row = src + long(__builtin_amdgcn_readlane(q, s * F::NRA + l));
+                const Tst *row = src + lane_offset(q, s * F::NRA + l);
                 xa[s][l].load(reinterpret_cast<const Tst *>(reinterpret_cast<const char *>(row) + tb));
             };
             if (wrap == 0) {
@@ -391,7 +395,7 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
                         const int k = s * F::NRA + l;
                         if (ALL || ((wrap >> k) & 1)) {
                             const int cap = __builtin_amdgcn_readlane(rcap, k);
-                            const Tst *row = src + long(__builtin_amdgcn_readlane(roff, k));
+                            const Tst *row = src + lane_offset(int(roff), k);
                             const int q0 = __builtin_amdgcn_readlane(rpos, k) + i, q1 = q0 + 1;
                             xa[s][l].set(row + (q0 - ((q0 >= cap) ? cap : 0)), row + (q1 - ((q1 >= cap) ? cap : 0)));
                             if constexpr (!ALL)
@@ -440,6 +444,10 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
                         }
                     }
                     const int k = 2 * lane - nv;
+                    if (t0 + nv == a.Tp) {
+                        // in place, a chunk of one tile writes where other lanes have just read
+                        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    }
                     if (t0 + nv == a.Tp && k >= 0 && k < F::OVA) {
 #pragma unroll
                         for (int l = 0; l < F::NRA; l++)
@@ -568,11 +576,11 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
             // part. The lane reads stay outside the branch on live: what is formed inside it is
             // formed for live lanes only, and lane 0 is not one.
             if (!__any(rpos + nv > rcap)) {
-                const int q = roff + rpos;
-                int qs[F::NRB];
+                const int q = int(roff + unsigned(rpos));
+                unsigned qs[F::NRB];
 #pragma unroll
                 for (int hp = 0; hp < F::NRB; hp++)
-                    qs[hp] = __builtin_amdgcn_readlane(q, hp);
+                    qs[hp] = lane_offset(q, hp);
                 if (live) {
 #pragma unroll
                     for (int hp = 0; hp < F::NRB; hp++)
@@ -582,7 +590,7 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
 #pragma unroll
                 for (int hp = 0; hp < F::NRB; hp++) {
                     const int cap = __builtin_amdgcn_readlane(rcap, hp);
-                    Tst *row = dst + long(__builtin_amdgcn_readlane(roff, hp));
+                    Tst *row = dst + lane_offset(int(roff), hp);
                     int q = __builtin_amdgcn_readlane(rpos, hp) + 2 * lane - F::OV;
                     q -= (q >= cap) ? cap : 0;
                     if (live)
@@ -633,21 +641,6 @@ k_stage2(Stage2Args a)
 }  // namespace
 
 
-long tree_state_nelts(int dd)
-{
-    switch (dd) {
-        case 1: return RegDims<1>::NSTATE;
-        case 2: return RegDims<2>::NSTATE;
-        case 3: return RegDims<3>::NSTATE;
-        case 4: return RegDims<4>::NSTATE;
-        case 5: return RegDims<5>::NSTATE;
-        case 6: return RegDims<6>::NSTATE;
-        case 7: return RegDims<7>::NSTATE;
-        case 8: return RegDims<8>::NSTATE;
-        default: return 0;
-    }
-}
-
 // Dynamic LDS above 64 KB (ranks 7 and 8) must be allowed per kernel; gfx950 allows 160 KB.
 static void allow_lds(const void *fn, int bytes)
 {
@@ -660,10 +653,9 @@ static void allow_lds(const void *fn, int bytes)
 // besides (launch, state). Takes the power of two with the shortest sum. One beam of rank 10
 // (32 instances x 22 tiles): stages 1 and 2 54 and 64 us in one segment, 13 and 12 us in 16; from some
 // 500 instances on, one segment.
-template<int DD>
+template<typename F>
 static int tree_nseg(long ninst, int Tp)
 {
-    using F = RegDims<DD>;
     constexpr int kStart = 2;
     constexpr long slots = 256L * cmin(16 / F::NW, 160 * 1024 / F::LDS_BYTES);
     const int ntiles = (Tp + F::U - 1) / F::U;
@@ -680,12 +672,42 @@ static int tree_nseg(long ninst, int Tp)
     return best;
 }
 
+// Calls f(RegDims<dd>()), dd = 1..8; r for other ranks.
+template<typename R, typename F>
+static R for_rank(int dd, R r, F f)
+{
+    switch (dd) {
+        case 1: return f(RegDims<1>());
+        case 2: return f(RegDims<2>());
+        case 3: return f(RegDims<3>());
+        case 4: return f(RegDims<4>());
+        case 5: return f(RegDims<5>());
+        case 6: return f(RegDims<6>());
+        case 7: return f(RegDims<7>());
+        case 8: return f(RegDims<8>());
+        default: return r;
+    }
+}
+
+int tree_segments(int dd, long ninst, int Tp)
+{
+    return for_rank(dd, 1, [&](auto d) { return tree_nseg<decltype(d)>(ninst, Tp); });
+}
+
+long tree_state_nelts(int dd, bool stage2, int nseg)
+{
+    return for_rank(dd, 0L, [&](auto d) { return long(d.nstate(stage2)) * (nseg > 1 ? 2 : 1); });
+}
+
+int tree_overlap(int dd)
+{
+    return for_rank(dd, 0, [](auto d) { return int(d.OVA); });
+}
+
 template<int DD, typename Args>
-static void launch_tree(void (*k)(Args), const Args &a0, hipStream_t st)
+static void launch_tree(void (*k)(Args), const Args &a, hipStream_t st)
 {
     using F = RegDims<DD>;
-    Args a = a0;
-    a.nseg = tree_nseg<DD>((1L << a.amb) * a.B, a.Tp);
     allow_lds((const void *) k, F::LDS_BYTES);
     hipLaunchKernelGGL(k, dim3(1 << a.amb, a.B, a.nseg), dim3(F::NW * 64), F::LDS_BYTES, st, a);
 }

@@ -53,7 +53,7 @@ struct Stage1Args {
     float *state;             // per (global beam, a): phase-A histories and line samples
     long state_bstride;       // per beam
     int B, amb, dd, Tp, beam0;
-    int nseg = 1;             // time segments (set by launch_stage1)
+    int nseg;                 // time segments: tree_segments()
     long chunk;               // chunk index (ring time = chunk*Tp + t)
     const long *chunk_dev = nullptr;   // if set, the chunk index is read here (graph replay)
 };
@@ -72,17 +72,18 @@ struct Stage2Args {
     float *state;             // per (global beam, j): phase-A histories and line samples
     long state_bstride;       // per beam
     int B, amb, dd, Tp, beam0;
-    int nseg = 1;             // time segments (set by launch_stage2)
+    int nseg;                 // time segments: tree_segments()
     long chunk;
     const long *chunk_dev = nullptr;   // if set, the chunk index is read here (graph replay)
 };
 
-// State per tree instance and chunk parity: tree_state_nelts(dd) floats. state_bstride holds two
-// parities: [parity][2^amb instances].
-long tree_state_nelts(int dd);
+// Time segments of a stage with ninst tree instances (2^amb times beams per batch), the same for every
+// chunk, and the floats of state per instance: twice with several segments, [chunk parity][2^amb instances].
+int tree_segments(int dd, long ninst, int Tp);
+long tree_state_nelts(int dd, bool stage2, int nseg);
 // Stage 2 reads a ring row from up to this many samples before the chunk's delayed start (phase
 // A's window).
-static constexpr int kTreeOverlap = 8;
+int tree_overlap(int dd);
 void launch_stage1(Dtype dt, const Stage1Args &a, hipStream_t st);
 void launch_stage2(Dtype dt, const Stage2Args &a, hipStream_t st);
 
