@@ -17,6 +17,8 @@
 #include "device_common.hpp"
 #include "kernels.hpp"
 
+#include <algorithm>
+
 namespace pirate_amd {
 
 template<typename Tout>
@@ -45,9 +47,13 @@ k_dequant(const void *data, const uint32_t *scoff, Tout *out, long nthreads)
 template<typename Tout>
 static void launch_dequant_t(const void *data, const void *scoff, void *out, long nsamples, hipStream_t st)
 {
-    const long nthreads = nsamples / (16 / long(sizeof(Tout)));
-    hipLaunchKernelGGL(k_dequant<Tout>, dim3((nthreads + 255) / 256), dim3(256), 0, st, data, (const uint32_t *) scoff,
-                       (Tout *) out, nthreads);
+    constexpr long V = 16 / long(sizeof(Tout));
+    // A launch takes less than 2^32 threads (of more, HIP runs the low 32 bits' worth, without an error).
+    for (long s0 = 0; s0 < nsamples; s0 += V << 30) {
+        const long nthreads = std::min(nsamples - s0, V << 30) / V;
+        hipLaunchKernelGGL(k_dequant<Tout>, dim3((nthreads + 255) / 256), dim3(256), 0, st, (const char *) data + s0 / 2,
+                           (const uint32_t *) scoff + s0 / 256, (Tout *) out + s0, nthreads);
+    }
 }
 
 void launch_dequant(Dtype dt, const void *data, const void *scoff, void *out, long nsamples, hipStream_t st)
