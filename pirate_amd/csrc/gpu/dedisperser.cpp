@@ -137,7 +137,6 @@ void GpuDedisperser::build_tables()
         }
 
         T.tpad = int(std::max(2 * t.pf.max_width, 4L));
-        T.nlev = std::max(integer_log2(t.pf.max_width), 1);
         // Rows start on 128-byte lines and the buffer is offset by 'lead' elements so that
         // chunk sample 0 (position tpad) of every row starts a line: the stage-2 tile stores
         // and the peak finder's loads then cover whole lines.
@@ -171,7 +170,7 @@ void GpuDedisperser::validate_gpu_limits()
         const TreeTables &T = tables[it];
         PDD_CHECK(t.dd_rank <= kGpuMaxDD, "GpuDedisperser: stage-2 dd_rank " << t.dd_rank << " not supported by pirate_amd (max " << kGpuMaxDD << ")");
         PDD_CHECK(t.pf.time_downsampling <= 512, "GpuDedisperser: time_downsampling too large");
-        PDD_CHECK(pf_config_supported(T.M, T.tpad, T.nlev, int(t.Dcore), int(t.pf.time_downsampling), t.nt_ds),
+        PDD_CHECK(pf_config_supported(T.M, T.tpad, int(t.Dcore), int(t.pf.time_downsampling), t.nt_ds),
                   "GpuDedisperser: tree " << it << ": peak-finder shape not supported (M=" << T.M << ")");
     }
 }
@@ -558,9 +557,13 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
     // stream p (0: st); st waits for every branch at the end. The branches p >= 1 start after tree
     // 0's stage 2 when its instances alone fill the chip, else right after the gridding: stage 1
     // and stage 2 of tree 0 then run near the HBM bandwidth on their own, and what the branches
-    // share best is the peak finder's time (16 beams x 16384 channels: late 5.44 ms, early
-    // 5.49 ms; float16 4.06 and 4.16 ms; rank 15 with subbands 5.32 and 5.58 ms). Small chains
-    // only gain from kernels side by side (2 beams of rank 8, 3 primary trees: 0.37 and 0.32 ms).
+    // share best is the peak finder's time. Medians, early and late, four primary trees, float32 and float16:
+    //   64 to 128 instances (1 beam of ranks 12, 14): 203, 231; 196, 207 us; 483, 525; 408, 442 us
+    //   256 to 512 (4 beams of ranks 12, 14): 447, 468; 355, 381 us; 1322, 1330; 986, 998 us
+    //   256 of rank 8 (1 beam of rank 16): 1520, 1504; 1337, 1302 us; of rank 15 with subbands 1838, 1794; 1535, 1454 us
+    //   1024 (8 beams of ranks 14, 15 with subbands): 2458, 2435; 1842, 1807 us; 6539, 6497; 5145, 4945 us
+    // So below 256 early wins by up to 14%, above it late by up to 6% for stages of ranks 7 and 8, while small
+    // ranks stay up to 10% faster early (64 beams of rank 8, float16: 311, 344 us).
     // tuning.fork == 2: every branch on 'st' in order (one kernel at a time, for per-kernel timing).
     const bool serial = (tuning.fork == 2);
     const bool full = (B << plan->stage1_dd_rank[0]) >= 256;      // stage-2 instances of tree 0, one per CU
@@ -676,7 +679,6 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
             f.M = T.M;
             f.N = T.N;
             f.P = int(t.nprofiles);
-            f.nlev = T.nlev;
             f.Tp = t.nt_ds;
             f.Dout = int(t.pf.time_downsampling);
             f.Dcore = int(t.Dcore);

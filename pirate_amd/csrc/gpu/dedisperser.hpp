@@ -164,7 +164,7 @@ public:
         std::vector<int> m_to_n;
         std::vector<int> nband, mband; // subband bands and first multiplet per level 0..pf_rank
         int flmax = 0;                 // largest subband final lag
-        int tpad = 0, nlev = 0, rowlen = 0, M = 0, N = 0;
+        int tpad = 0, rowlen = 0, M = 0, N = 0;
         int lead = 0;                  // element offset of the peak-finder rows in their buffer
     };
     std::vector<TreeTables> tables;

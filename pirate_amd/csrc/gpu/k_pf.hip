@@ -49,9 +49,8 @@ __host__ __device__ constexpr int pf_tile_len(int dout)
     return (dout >= 4) ? ((dout > kPfTileMin) ? dout : kPfTileMin) : 8 * dout;
 }
 
-bool pf_config_supported(int M, int tpad, int nlev, int Dcore, int Dout, int Tp)
+bool pf_config_supported(int M, int tpad, int Dcore, int Dout, int Tp)
 {
-    (void) nlev;
     if (M < 1 || M > kPfThreads || Dout < 1 || Dout > kPfMaxDout || (Dout & (Dout - 1)))
         return false;
     if (tpad % 4)

@@ -27,14 +27,14 @@
 // consecutive samples, and the first OVA = 2^K1 (phase A) or OV = 2^K2 (phase B) samples of a
 // window come before the tile and only feed the lags. So there are no histories to hold or to
 // select from, and a shift by L and L + 1 together takes 3 lane moves for two samples instead of
-// 4. 96 samples fill 52 to 56 of 64 lanes, tiles of 64 no more than 40.
+// 4. A window of 96 samples fills 48 to 56 of 64 lanes (rank 1 to rank 7), one of 64 no more than 40.
 //   Rank 8 has LDS for tiles of 64 to 80 samples only; there phase A holds lane = one sample,
 // with lanes t < L taking the previous tile's values (tree_regs.hpp).
 // Between the phases a row goes through an LDS line that holds its last lag + OV samples and the
 // current tile; phase A appends at the end, phase B reads the OV + U samples at the start and
-// moves the line down by U. The lines persist across chunks in an HBM state buffer,
-// double-buffered by chunk parity, with the last OVA input samples of stage 1 (stage 2 finds
-// its own in the ring, whose rows are OVA samples longer) or rank 8's histories.
+// moves the line down by U. The lines persist across chunks in an HBM state buffer (twice, by chunk
+// parity, where a chunk has several time segments), with the last OVA input samples of stage 1 (stage
+// 2 finds its own in the ring, whose rows are OVA samples longer) or rank 8's histories.
 //
 // A chunk that is no multiple of U ends in a smaller tile (a multiple of 32 samples): its loads
 // stay inside the chunk, its stores stop at the chunk's end, and the lines move down by its

@@ -113,7 +113,7 @@ struct PfArgs {
     void *out_max;            // (B, ndm_out, nt_out), storage dtype
     unsigned int *out_argmax; // (B, ndm_out, nt_out)
     long out_bstride;
-    int B, ndm_out, M, N, P, nlev, Tp, Dout, Dcore, ndm_wt, nt_wt, nt_out;
+    int B, ndm_out, M, N, P, Tp, Dout, Dcore, ndm_wt, nt_wt, nt_out;
     int beam0;                // global index of the batch's first beam (sb rows are per global beam)
     int nseg = 1;             // time segments per chunk (set by launch_pf)
     int two_step = -1;        // two-step kernel: -1 by launch_pf's rule, 0 never, 1 wherever there is one
@@ -121,7 +121,7 @@ struct PfArgs {
     double *out_var = nullptr;   // optional (B, ndm_out, M, P) float64: per-chunk mean square of each
                                  // (multiplet, profile)'s weighted candidates
 };
-bool pf_config_supported(int M, int tpad, int nlev, int Dcore, int Dout, int Tp);
+bool pf_config_supported(int M, int tpad, int Dcore, int Dout, int Tp);
 void launch_pf(Dtype dt, const PfArgs &a, hipStream_t st);
 
 }  // namespace pirate_amd

@@ -1,4 +1,4 @@
-// Register-resident sub-trees shared by the tree kernels (gfx950).
+// Register-resident sub-trees with pass histories: phase A of the rank-8 tree kernels (gfx950).
 //
 // A rank-K sub-tree over 2^K rows holds one row per register, lane = time sample of a
 // 64-sample tile. Pass r pairs rows e = fout*2^(r+1) + dmb and o = e + 2^r (dmb < 2^r):
@@ -82,7 +82,7 @@ __device__ __forceinline__ void load_hist(float (&h)[Sub<K>::NH], const float *s
 }
 
 // Saves the last 2^r samples of each pass history; 'hi' = valid lanes of the last tile
-// (64, or 32 for a half tile).
+// (64, or 32 at the end of a chunk of an odd number of 32 samples).
 template<int K>
 __device__ __forceinline__ void save_hist(const float (&h)[Sub<K>::NH], float *dst, int lane, int hi)
 {
