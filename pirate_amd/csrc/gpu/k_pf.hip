@@ -828,10 +828,13 @@ static bool pf_two_step(const PfArgs &a, long nblocks, int TL)
 }
 
 // Time segments per chunk, of whole tiles and at least nwarm of them (see rotate_rows). One step: the
-// fewest that give at least a.target_blocks workgroups (2048 unless tuned). Two steps: up to that number, the one
-// with the shortest rounds of resident workgroups (three per CU) times tiles walked, warm-up
-// among them: with 32 workgroups of 1024 float32 samples 16 segments take 24 us, 32 segments (64 positions walked
-// for 32) 33 us; 512 workgroups of 2048 samples, 3 segments 279 us, 6 segments 277, 8 288 us. With out_var, one segment.
+// fewest that give at least a.target_blocks workgroups (2048 unless tuned). Two steps: up to that
+// number, the count that is done first, a workgroup's time being its tiles and the warm-up's
+// times a factor for its company on the CU (three of 768 run there at a time), and rounds of 768 running into
+// each other. The factors are fitted to 170 launches of 8 to 2344 workgroups (in one segment) in all types: 1.3% from the best
+// count on average, 20% at most. 32 workgroups of 1024 float32
+// samples: 16 segments 24 us, 32 (64 positions walked for 32) 33 us; 256 of 1024: 3 segments 77 us, 4 94, 8 88 us;
+// 512 of 2048 float16 samples: 1, 2, 4 and 8 segments 264, 240, 224 and 244 us. With out_var, one segment.
 static int pf_nseg(const PfArgs &a, bool two_step, long nblocks, int TL)
 {
     if (a.out_var)
@@ -841,9 +844,12 @@ static int pf_nseg(const PfArgs &a, bool two_step, long nblocks, int TL)
     if (!two_step)
         return most;
     int best = 1;
-    long cost = 0;
+    double cost = 0.0;
     for (int n = 1; n <= most; n++) {
-        const long c = ((nblocks * n + 767) / 768) * ((ntiles + n - 1) / n + nwarm);
+        const long nwg = nblocks * n;
+        const double w = nwg / 768.0;
+        const double c = ((ntiles + n - 1) / n + nwarm) * ((nwg <= 256) ? 0.6 : (nwg <= 512) ? 0.85 : (nwg <= 768) ? 1.0
+                                                           : 0.34 * w + 0.51 * ((nwg + 767) / 768) + 0.21);
         if (n == 1 || c < cost) {
             best = n;
             cost = c;
