@@ -802,20 +802,23 @@ static void launch_pf_lw(const PfArgs &a, hipStream_t st, dim3 grid)
 }
 
 // Two steps or one. Step 2 walks NBACK + 1 bins per output bin, spread over the M multiplets of a DM
-// row, so it pays with many multiplets and long bins. Medians of kernel times, one step and two, us:
-//   (NBACK + 1) / M   one    two    (2048 samples, float32 and float16)
-//   0.12, M 16        112    81     109    68       boxcars up to 4, bins of 16
-//   0.31, M 16        130    104    125    94       16, bins of 8
-//   0.62, M 8         126    109    122    102      16, bins of 8
-//   1.12, M 8         135    150    127    128      32, bins of 8
-//   2.25, M 4         84     97     75     82       16, bins of 4
-//   4.25, M 4         97     186    85     125      32, bins of 4
+// row, so it pays with many multiplets and long bins. One step and two, each at its best segment count, us,
+// 2048 samples, float32 and float16:
+//   (NBACK + 1) / M                                    float32      float16
+//   0.12  (M 16, boxcars up to 4, bins of 16)          101    70     96    60
+//   0.31  (M 16, 16, bins of 8)                        122    95    113    86
+//   0.62  (M 8, 16, bins of 8)                         117   105    109    98
+//   1.12  (M 8, 32, bins of 8)                         130   133    120   119
+//   2.25  (M 4, 16, bins of 4)                          80    96     69    80
+//   4.25  (M 4, 32, bins of 4)                          91   178     79   125
 // Bins of 4 went from 27% slower to 20% faster and seldom occur with 16 multiplets or more; bins of 1
 // and 2 were up to 3.2 times slower, and with bins of 32 the unrolled walks spill (up to 7 times slower).
 // Small launches are bounded by latency: the tiles of one step are shorter, those of two steps pass
 // without a barrier, which counts more the longer the warm-up is. Up to 2^14 positions of a
 // workgroup's chunk and boxcars of 2 to 8 samples, one step took 9 to 16 us and two steps 13 to 19;
-// with boxcars of 16 and 32 16 and 29 against 14 and 27 (float16 17 and 23).
+// with boxcars of 16 and 32 16 and 29 against 14 and 27 (float16 17 and 23). So between 0.7 and 1.15 two steps are
+// taken for long boxcars and up to 2^17 positions: 2^15, boxcars of 32, 31 and 27 us (float16 29 and 23); 2^18
+// as above; 2^20 455 and 500 us (float16 408 and 425).
 static bool pf_two_step(const PfArgs &a, long nblocks, int TL)
 {
     if (a.out_var || !pf_has_two_step(a.Dout) || a.Tp % TL != 0 || a.two_step == 0)
@@ -824,7 +827,9 @@ static bool pf_two_step(const PfArgs &a, long nblocks, int TL)
         return true;
     const int wmax = 1 << ((a.P - 1) / 3);
     const int bins = (a.tpad + a.Dout - 1) / a.Dout + 1;       // NBACK + 1
-    return 10 * bins <= 7 * a.M && (wmax >= 16 || nblocks * a.Tp > (1 << 14));
+    const long work = nblocks * a.Tp;
+    return (10 * bins <= 7 * a.M && (wmax >= 16 || work > (1 << 14)))
+           || (20 * bins <= 23 * a.M && wmax >= 16 && work <= (1 << 17));
 }
 
 // Time segments per chunk, of whole tiles and at least nwarm of them (see rotate_rows). One step: the
