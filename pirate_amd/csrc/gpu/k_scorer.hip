@@ -149,8 +149,11 @@ __device__ __forceinline__ void store_act(ushort_t *out, int t, int q, f32x4 acc
 
 // Layers 1..3 of the wave's four column blocks; y3[i][r] = Y_3[co = 4q + r][t = 16(4w + i) + l % 16].
 // Barriers: the caller has synchronized after load_tile; A1t and A2t are complete on return.
-__device__ void forward_layers(const ushort_t *Xt, ushort_t *A1t, ushort_t *A2t, const s16x4 *Wf,
-                               const float *bias1, const float *bias2, const float *bias3, float y3[4][4])
+// Marked used: its one caller is the training kernel, and specialized for that caller's arguments it
+// takes 18 more LDS reads and 14 more registers there (65536 tiles 7.95 ms instead of 7.52).
+__device__ __attribute__((used)) void forward_layers(const ushort_t *Xt, ushort_t *A1t, ushort_t *A2t,
+                                                     const s16x4 *Wf, const float *bias1, const float *bias2,
+                                                     const float *bias3, float y3[4][4])
 {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6, m = l & 15, q = l >> 4;
     for (int i = 0; i < 4; i++) {
