@@ -502,13 +502,13 @@ k_pf_one(PfArgs a)
         rotate_rows(rows, nstreams, a);
 }
 
-// The peak finder proper, in two steps. Step 1 walks every stream once and keeps per bin only
+// Two steps (bins of 8 and 16 samples; pf_two_step says where). Step 1 walks every stream once and keeps per bin only
 // the largest value of each profile (PfMax: about 1.5 maxima per candidate in place of a
 // multiply, a compare and two selects), weights these, and leaves the stream's largest value
 // and its first level in LDS. Step 2 runs once per kPfBatch bins, one lane per (DM row, bin):
 // it picks the winning multiplet (largest value, then first (level, m)) and walks that one
 // stream over the bin again with PfLane, which gives the value and the token of the first
-// maximum. A DM row has M streams, so step 2 costs 1/M of a full walk per stream.
+// maximum. A DM row has M streams, so step 2 costs (NBACK + 1) / M of a full walk per stream.
 // Infinities, NaN and samples that could make a sum overflow (pf_wild): a stream is marked in each
 // bin whose windows hold one. A wave with a marked lane walks that bin with PfLane in place of
 // PfMax, from the same windows, and leaves value and token for step 2, which then walks nothing
@@ -523,10 +523,11 @@ k_pf_one(PfArgs a)
 // instruction writes the i-th 16 bytes, so the 16-byte chunks of a row are permuted on the
 // global side (slot s of row r holds chunk s ^ (r & 7)), and the 16-byte reads of 8
 // neighbouring rows cover all banks. 51 KB of LDS and 168 VGPRs: three workgroups (12 waves)
-// per CU. Bounded by VALU issue (about 400 instructions per stream and 16-sample bin at Wmax 16,
-// against 520 with every candidate compared) and, for float32, near half by the row reads.
-// 16384 DM rows x 2048 samples x 16 beams, Wmax 16, bins of 16: float32 0.774 -> 0.547 ms,
-// float16 0.736 -> 0.422 ms; 36 multiplets, 8 beams of rank 15, float16: 2.28 -> 1.01 ms.
+// per CU. Bounded by VALU issue (475 instructions per stream and 16-sample bin at Wmax 16, step 2 and
+// warm-up included, against 770 with every candidate compared) and, for float32, near half by the row reads.
+// 16384 DM rows x 2048 samples x 16 beams, Wmax 16, bins of 16: float32 0.774 -> 0.541 ms,
+// float16 0.736 -> 0.423 ms; 36 multiplets, 8 beams of rank 15, float16: 2.28 -> 1.01 ms. No instance
+// spills vector registers; all keep 4 to 58 scalars in lanes of one, outside a bin's walk.
 // Tried: tiles of 16 positions staged through registers (each 128-byte line fetched twice,
 // float32 0.93 ms), two staging buffers and 8 waves per CU (0.68 ms), the walk's float32 loads
 // all at once with bins of 16 (31 registers spilled, 1.31 ms).

@@ -272,7 +272,7 @@ __device__ __forceinline__ void load_bias(const float *P, int o, int q, float *b
 // and written to LDS when layer 1 has read this tile's, and the pooled channels of a tile are
 // combined by one wave while the others start the next tile: three barriers per tile. Every
 // product is accumulated in the order of the training kernel's forward pass, so both give the
-// same bits. 8192 bf16 tiles: 131 us; with the fragments read from LDS for every product, one
+// same bits. 8192 bf16 tiles: 130 to 140 us; with the fragments read from LDS for every product, one
 // work group per CU and scalar row loads, 555 us.
 //
 // X rows hold their 64 channels so that the 16 bytes of lane group q are channels 4q..4q+3 of two
