@@ -344,8 +344,8 @@ void GpuDedisperser::allocate()
             host_bytes_allocated += hb;
         }
         s1_nseg[p] = tree_segments(dd1, pow2(amb1) * B, int(Tp));
-        s1_state_bstride[p] = pow2(amb1) * tree_state_nelts(dd1, false, s1_nseg[p]);
-        s1_state[p] = dalloc(size_t(total_beams) * s1_state_bstride[p] * sizeof(float));
+        s1_state_bstride[p] = pow2(amb1) * tree_state_nelts(dd1, false);
+        s1_state[p] = dalloc(size_t(total_beams + (s1_nseg[p] > 1 ? nstreams * B : 0)) * s1_state_bstride[p] * sizeof(float));
     }
 
     stage2_lags.resize(ntrees);
@@ -375,8 +375,8 @@ void GpuDedisperser::allocate()
         sb[it] = dalloc((size_t(total_beams) * t.ndm_out * T.M * T.rowlen + T.lead) * elt_bytes);
         d_m_to_n[it] = up_int(T.m_to_n);
         s2_nseg[it] = tree_segments(t.dd_rank, pow2(t.amb_rank) * B, int(t.nt_ds));
-        s2_state_bstride[it] = pow2(t.amb_rank) * tree_state_nelts(t.dd_rank, true, s2_nseg[it]);
-        s2_state[it] = dalloc(size_t(total_beams) * s2_state_bstride[it] * sizeof(float));
+        s2_state_bstride[it] = pow2(t.amb_rank) * tree_state_nelts(t.dd_rank, true);
+        s2_state[it] = dalloc(size_t(total_beams + (s2_nseg[it] > 1 ? nstreams * B : 0)) * s2_state_bstride[it] * sizeof(float));
         weights[it] = dalloc(size_t(nbatches_wt) * B * t.ndm_wt * t.nt_wt * t.nprofiles * T.N * sizeof(float));
         // out_max / out_argmax: views into the output region (below)
         out_max[it].nbytes = size_t(nbatches_out) * B * t.ndm_out * t.nt_out * elt_bytes;
@@ -570,6 +570,14 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
     const bool late_fork = (tuning.fork < 0) ? full : (tuning.fork == 1);
     if (!late_fork && !serial)
         HIP_CHECK(hipEventRecord(ev_fork_s, st));
+    auto set_state = [&](StateArgs &a, const DeviceArray &state, long bstride, int nseg) {
+        a.state = (float *) state.ptr;
+        a.state_bstride = bstride;
+        a.nbatches = int(nbatches);
+        a.nspare = (nseg > 1) ? int(nstreams) : 0;
+        a.batch = int(ibatch);
+        a.blocks = a.blocks_of(ichunk);
+    };
     for (long p = 0; p < npri; p++) {
         hipStream_t sp = (p && !serial) ? bstreams[p] : st;
         if (sp != st)
@@ -582,8 +590,7 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
         s.ring.row_off = (const long *) ring1_row_off[p].ptr;     // spilled rows: the outbox
         s.ring.row_cap = (const long *) ring1_row_cap[p].ptr;
         s.ring.bstride = ring_bstride[p];
-        s.state = (float *) s1_state[p].ptr;
-        s.state_bstride = s1_state_bstride[p];
+        set_state(s, s1_state[p], s1_state_bstride[p], s1_nseg[p]);
         s.nseg = s1_nseg[p];
         s.B = int(B);
         s.amb = int(plan->stage1_amb_rank[p]);
@@ -623,8 +630,7 @@ void GpuDedisperser::launch_chain(const void *input, long ichunk, long ibatch, l
                 s2.nband[lev] = (lev < T.nband.size()) ? T.nband[lev] : 0;
                 s2.mband[lev] = (lev < T.mband.size()) ? T.mband[lev] : 0;
             }
-            s2.state = (float *) s2_state[it].ptr;
-            s2.state_bstride = s2_state_bstride[it];
+            set_state(s2, s2_state[it], s2_state_bstride[it], s2_nseg[it]);
             s2.nseg = s2_nseg[it];
             s2.B = int(B);
             s2.amb = t.amb_rank;

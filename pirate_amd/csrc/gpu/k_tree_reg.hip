@@ -32,8 +32,7 @@
 // with lanes t < L taking the previous tile's values (tree_regs.hpp).
 // Between the phases a row goes through an LDS line that holds its last lag + OV samples and the
 // current tile; phase A appends at the end, phase B reads the OV + U samples at the start and
-// moves the line down by U. The lines persist across chunks in an HBM state buffer (twice, by chunk
-// parity, where a chunk has several time segments), with the last OVA input samples of stage 1 (stage
+// moves the line down by U. The lines persist across chunks in an HBM state buffer, with the last OVA input samples of stage 1 (stage
 // 2 finds its own in the ring, whose rows are OVA samples longer) or rank 8's histories.
 //
 // A chunk that is no multiple of U ends in a smaller tile (a multiple of 32 samples): its loads
@@ -274,12 +273,10 @@ __device__ __forceinline__ void reg_tree_body(const Args &a)
     const int first = int(blockIdx.z) * ntiles / a.nseg, end = (int(blockIdx.z) + 1) * ntiles / a.nseg;
     const int start = blockIdx.z ? first - F::WARM : 0;       // >= 0: the host checks it
 
-    // state: one segment reads and writes it in place, several keep it twice by chunk parity (segment
-    // 0 reads what the last one writes)
-    const long half_state = (a.nseg > 1) ? a.state_bstride >> 1 : 0;
-    float *st = a.state + gbeam * a.state_bstride + long(tr) * F::nstate(STAGE2);
-    const float *rd = st + (chunk & 1) * half_state;
-    float *wr = st + ((chunk + 1) & 1) * half_state;
+    const StateBlocks blocks = a.chunk_dev ? a.blocks_of(chunk) : a.blocks;
+    float *st = a.state + b * a.state_bstride + long(tr) * F::nstate(STAGE2);
+    const float *rd = st + blocks.rd * a.B * a.state_bstride;
+    float *wr = st + blocks.wr * a.B * a.state_bstride;
 
     // this wave's phase-B sub-tree j: bitrev(j), its lines, and sum of bitrev(j') over j' < j
     const int j = wid, bj = __builtin_amdgcn_readfirstlane(bitrev_dev(j, F::K1));
@@ -694,9 +691,9 @@ int tree_segments(int dd, long ninst, int Tp)
     return for_rank(dd, 1, [&](auto d) { return tree_nseg<decltype(d)>(ninst, Tp); });
 }
 
-long tree_state_nelts(int dd, bool stage2, int nseg)
+long tree_state_nelts(int dd, bool stage2)
 {
-    return for_rank(dd, 0L, [&](auto d) { return long(d.nstate(stage2)) * (nseg > 1 ? 2 : 1); });
+    return for_rank(dd, 0L, [&](auto d) { return long(d.nstate(stage2)); });
 }
 
 int tree_overlap(int dd)

@@ -46,12 +46,30 @@ struct RingView {
     long bstride;             // elements per beam
 };
 
-struct Stage1Args {
+// State blocks, [B beams][2^amb instances] each, that a launch reads and writes: its batch's with one
+// time segment. With several, segment 0 reads what the last one writes; then there are nspare more, one per stream.
+// Launch n (of the batches in turn, on stream n % nspare) writes the block that the launch nspare before
+// it, on the same stream, read, and reads the one written nbatches launches before it.
+struct StateBlocks {
+    long rd, wr;
+};
+
+struct StateArgs {
+    float *state;             // phase-A histories and line samples
+    long state_bstride;       // per beam
+    int nbatches, nspare, batch;
+    StateBlocks blocks;       // blocks_of(chunk), unless the chunk index is read on the device
+    __host__ __device__ StateBlocks blocks_of(long chunk) const
+    {
+        const unsigned long launch = (unsigned long) (chunk) * nbatches + batch, n = nbatches + nspare;
+        return nspare ? StateBlocks{long((launch + nspare) % n), long(launch % n)} : StateBlocks{batch, batch};
+    }
+};
+
+struct Stage1Args : StateArgs {
     const void *in;
     long in_bstride;
     RingView ring;
-    float *state;             // per (global beam, a): phase-A histories and line samples
-    long state_bstride;       // per beam
     int B, amb, dd, Tp, beam0;
     int nseg;                 // time segments: tree_segments()
     long chunk;               // chunk index (ring time = chunk*Tp + t)
@@ -62,15 +80,13 @@ struct Stage1Args {
 // ---- stage-2 tree + subband streams -> peak-finder input rows ----
 // pf_rank = (dd + 1) / 2; band counts and first multiplets per subband level 0..pf_rank.
 static constexpr int kMaxPfRank = 4;
-struct Stage2Args {
+struct Stage2Args : StateArgs {
     RingView ring;            // ring of the tree's primary tree
     const int *row_lag;       // (2^dd rows fc, 2^amb j) -> lag, indexed fc*2^amb + j
     void *sb;                 // (B, ndm_out, M, rowlen) peak-finder input rows
     long sb_bstride;
     int rowlen, tpad, M;
     int nband[kMaxPfRank + 1], mband[kMaxPfRank + 1];
-    float *state;             // per (global beam, j): phase-A histories and line samples
-    long state_bstride;       // per beam
     int B, amb, dd, Tp, beam0;
     int nseg;                 // time segments: tree_segments()
     long chunk;
@@ -78,9 +94,9 @@ struct Stage2Args {
 };
 
 // Time segments of a stage with ninst tree instances (2^amb times beams per batch), the same for every
-// chunk, and the floats of state per instance: twice with several segments, [chunk parity][2^amb instances].
+// chunk, and the floats of state per instance.
 int tree_segments(int dd, long ninst, int Tp);
-long tree_state_nelts(int dd, bool stage2, int nseg);
+long tree_state_nelts(int dd, bool stage2);
 // Stage 2 reads a ring row from up to this many samples before the chunk's delayed start (phase
 // A's window).
 int tree_overlap(int dd);

@@ -8,19 +8,20 @@ from gpu_cases import BASE, chord16k_with_beams, pt
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize('dtype,limit', [('float32', 1.500), ('float16', 0.767)])
-def test_bytes_per_beam(dtype, limit):
-    """16384 channels, four primary trees: what each beam beyond the first 16 takes (GiB). The chain's
-    trees run in one time segment here and hold one copy of their state."""
+@pytest.mark.parametrize('dtype,batch,limit', [('float32', 0, 1.500), ('float16', 0, 0.767), ('float32', 2, 1.195), ('float16', 2, 0.614)])
+def test_bytes_per_beam(dtype, batch, limit):
+    """16384 channels, four primary trees: what each beam beyond the first 16 takes (GiB), all beams in
+    one batch and in batches of 2, whose trees run in several time segments."""
     import pirate_amd as pa
 
     def nbytes(n):
-        dd = pa.GpuDedisperser(pa.DedispersionPlan(pa.DedispersionConfig.from_dict(dict(chord16k_with_beams(n), dtype=dtype))))
+        cfg = dict(chord16k_with_beams(n, batch), dtype=dtype, num_active_batches=2 if batch else 1)
+        dd = pa.GpuDedisperser(pa.DedispersionPlan(pa.DedispersionConfig.from_dict(cfg)))
         dd.allocate()
         return dd.gpu_bytes()
 
     per_beam = (nbytes(32) - nbytes(16)) / 16 / 2**30
-    print(f'[memory] {dtype}: {per_beam:.5f} GiB per beam', flush=True)
+    print(f'[memory] {dtype} {batch}: {per_beam:.5f} GiB per beam', flush=True)
     assert per_beam <= limit
 
 
